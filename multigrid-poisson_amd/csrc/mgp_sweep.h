@@ -21,6 +21,13 @@ template <class T>
 int march_sweep2(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_array* f, const mgp_faces* faces,
                  const int64_t box[6], double omega, void* stream, const mgp_array* coarse = nullptr,
                  bool zero_in = false);
+// one or two sweeps through workgroup tiles (mgp_tile.hip; arguments as
+// march_sweep / march_sweep2); MGP_ERR_ARG where the level or the layouts do
+// not allow it
+template <class T>
+int tile_sweep(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_array* f, const mgp_faces* faces,
+               const int64_t box[6], double omega, int sweeps, void* stream, const mgp_array* coarse, bool zero_in);
+extern int64_t g_tile;
 extern int64_t g_sweep_pair;
 extern int64_t g_sweep2_rows;
 extern int64_t g_sweep2_prolong;

@@ -34,6 +34,7 @@
 #include "mgp_device.h"
 #include "mgp_point.h"
 #include "mgp_sweep.h"
+#include "mgp_wave.h"
 
 namespace mgp {
 
@@ -61,10 +62,11 @@ static inline int64_t target_wgs(int64_t own) { return own > 0 ? own : g_sweep_t
 int64_t g_small_points = 1 << 18;
 int64_t g_small_min_chunk = 1;
 // the Gauss-Seidel smoother pairs its sweeps (mgp_rbgs_sweep2_*) on levels of
-// at least this many points; below it two one-pass sweeps are faster (FP64:
-// 257 x 257 x 129 pair 228 us, two sweeps 169 us; 513 x 513 x 257 pair
-// 0.83 ms, two sweeps 0.94 ms)
-int64_t g_pair_min_points = 1 << 25;
+// at least this many points (workgroup tiles, FP64: 257 x 257 x 129 pair 84 us,
+// two sweeps 104 us; 129 x 129 x 65 pair 36 us, two sweeps 32 us, but with the
+// correction inside 44 us against 46 us and one launch less; 65 x 65 x 33 pair
+// 24 us, two sweeps 21 us)
+int64_t g_pair_min_points = 1 << 20;
 extern int64_t g_sweep_min_chunk;
 static inline int64_t min_chunk_for(int64_t points) {
     return points < g_small_points ? g_small_min_chunk : g_sweep_min_chunk;
@@ -80,78 +82,6 @@ constexpr int TY = RH - 2;    // interior rows per tile
 constexpr int UW = RW + 2;    // old-plane rectangle (2-point ring) width
 constexpr int UH = RH + 2;    // ... height
 constexpr int NBORDER = 2 * UW + 2 * RH;  // outermost ring of the old-plane rectangle
-
-template <class T>
-struct MarchArgs {
-    View<T> ui, uo, f;
-    View<T> c;  // coarse level whose prolongation the pass adds first (two-sweep pass only)
-    const T* g[6];
-    T two_h;
-    int64_t bx0, bx1, by0, by1, bz0, bz1;
-    int64_t lin0;
-    T one_omega, omega_sixth, hsq;
-    int ytiles, ztiles, ntiles, ntiles_pad;
-    int64_t xchunk;
-};
-
-// The shape points outside the box, copied from ui to uo by extra blocks of a
-// sweep launch (the blocks after the tiles): an out-of-place pass then leaves
-// a complete image of what the in-place half-sweeps leave, whichever of the
-// two buffers ends up current (the boundary points' own history of updates,
-// signs of zero included, stays with the solution).  The halo is not copied:
-// ghost values are formed again before every use.
-constexpr int COPY_PER_THREAD = 8;
-
-template <class T>
-inline int64_t complement_points(const View<T>& u, const int64_t b[6]) {
-    const int64_t BX = b[1] - b[0], BY = b[3] - b[2];
-    return (b[0] + u.n0 - b[1]) * u.n1 * u.n2 + BX * (b[2] + u.n1 - b[3]) * u.n2 + BX * BY * (b[4] + u.n2 - b[5]);
-}
-template <class T>
-inline int complement_blocks(const View<T>& u, const int64_t b[6], int threads) {
-    const int64_t per = (int64_t)threads * COPY_PER_THREAD;
-    return (int)((complement_points(u, b) + per - 1) / per);
-}
-
-// points [blk * blockDim * COPY_PER_THREAD, ...) of the complement, in the
-// order: x outside the box (whole planes), then y outside (box planes), then
-// z outside (box rows); consecutive threads take consecutive z where it runs.
-// PRO: ui + P(coarse) instead of ui (the pass that adds the prolongation);
-// ZERO: 0 (the pass whose input is zero and not read)
-template <class T, bool PRO = false, bool ZERO = false>
-__device__ __forceinline__ void copy_complement(const MarchArgs<T>& A, int blk) {
-    const int64_t n0 = A.ui.n0, n1 = A.ui.n1, n2 = A.ui.n2;
-    const int64_t BX = A.bx1 - A.bx0, BY = A.by1 - A.by0;
-    const int64_t xo = A.bx0 + n0 - A.bx1, yo = A.by0 + n1 - A.by1, zo = A.bz0 + n2 - A.bz1;
-    const int64_t c1 = xo * n1 * n2, c2 = BX * yo * n2, c3 = BX * BY * zo;
-    const int64_t per = (int64_t)blockDim.x * COPY_PER_THREAD;
-    const int64_t end = min(c1 + c2 + c3, (int64_t)(blk + 1) * per);
-    for (int64_t t = (int64_t)blk * per + threadIdx.x; t < end; t += blockDim.x) {
-        int64_t x, y, z;
-        if (t < c1) {
-            const int64_t a = t / (n1 * n2), r = t % (n1 * n2);
-            x = a < A.bx0 ? a : A.bx1 + (a - A.bx0);
-            y = r / n2;
-            z = r % n2;
-        } else if (t < c1 + c2) {
-            const int64_t u = t - c1, a = u / (yo * n2), r = u % (yo * n2), c = r / n2;
-            x = A.bx0 + a;
-            y = c < A.by0 ? c : A.by1 + (c - A.by0);
-            z = r % n2;
-        } else {
-            const int64_t u = t - c1 - c2, a = u / (BY * zo), r = u % (BY * zo), c = r % zo;
-            x = A.bx0 + a;
-            y = A.by0 + r / zo;
-            z = c < A.bz0 ? c : A.bz1 + (c - A.bz0);
-        }
-        if (ZERO)
-            A.uo.at(x, y, z) = (T)0;
-        else if (PRO)
-            A.uo.at(x, y, z) = A.ui.at(x, y, z) + trilinear<T>(A.c, x, y, z);
-        else
-            A.uo.at(x, y, z) = A.ui.at(x, y, z);
-    }
-}
 
 // element at a 32-bit byte offset from a wave-uniform base: lets the compiler
 // use the scalar-base + 32-bit vector-offset addressing form
@@ -451,67 +381,6 @@ __global__ void __launch_bounds__(64 * (RH / NQ)) k_rbgs_march(MarchArgs<T> A) {
 // value until their own update one step later), which is exactly what each
 // half-sweep's stencil reads.
 constexpr int WZ = 60;  // interior columns per wave tile
-
-// DPP lane move of a 32- or 64-bit value with bound_ctrl: a lane whose source
-// lane lies outside the wave reads 0.  No old value is involved, so the
-// compiler emits no initialising move before each DPP move.
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double v) {
-    typedef int i32x2 __attribute__((ext_vector_type(2)));
-    i32x2 w = __builtin_bit_cast(i32x2, v);
-    w.x = __builtin_amdgcn_mov_dpp(w.x, CTRL, 0xf, 0xf, true);
-    w.y = __builtin_amdgcn_mov_dpp(w.y, CTRL, 0xf, 0xf, true);
-    return __builtin_bit_cast(double, w);
-}
-template <class T>
-__device__ __forceinline__ T lane_prev(T v) {  // value of lane l-1 (z - 1); 0 on lane 0
-    return dpp_move<0x138>(v);                 // wave_shr:1
-}
-template <class T>
-__device__ __forceinline__ T lane_next(T v) {  // value of lane l+1 (z + 1); 0 on lane 63
-    return dpp_move<0x130>(v);                 // wave_shl:1
-}
-
-// Buffer-resource access (SGPR descriptor + 32-bit lane offset + SGPR row
-// offset): no per-lane address arithmetic.  A lane offset at or beyond the
-// record count drops the store in hardware, which masks stores without
-// branches; only the lane (VGPR) offset is used for that, since the range
-// check does not cover the SGPR offset.  Loads always use in-range offsets.
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-constexpr uint32_t BUF_OOB = 0x40000000u;  // offset past any plane (planes < 1 GiB)
-// cache-policy bits of the buffer loads and stores (gfx950: bit 0 sc0, bit 1
-// nt, bit 4 sc1); a build-time choice, measured per kernel
-#ifndef MGP_LOAD_POLICY
-#define MGP_LOAD_POLICY 0
-#endif
-#ifndef MGP_STORE_POLICY
-#define MGP_STORE_POLICY 0
-#endif
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void* base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-template <class T>
-__device__ __forceinline__ T bload(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff);
-template <>
-__device__ __forceinline__ double bload<double>(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, MGP_LOAD_POLICY));
-}
-template <>
-__device__ __forceinline__ float bload<float>(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, MGP_LOAD_POLICY));
-}
-__device__ __forceinline__ void bstore(double v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)voff, (int)soff, MGP_STORE_POLICY);
-}
-__device__ __forceinline__ void bstore(float v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, (int)voff, (int)soff,
-                                          MGP_STORE_POLICY);
-}
 
 // EDGE: the tile has rows outside the box or in-plane Neumann ghost positions
 // (boundary tiles only); the other tiles run a copy of the loop without the
@@ -2008,6 +1877,10 @@ __global__ void __launch_bounds__(64) k_resid_fw_wave(RFArgs<T> A) {
 template <class T>
 int march_sweep(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_array* f, const mgp_faces* faces,
                 const int64_t b[6], double omega, int64_t xchunk, void* stream) {
+    if (g_sweep_kernel == 2 && g_sweep_rows == 0 && g_sweep_depth == 1) {
+        const int rc = tile_sweep<T>(mode, ui, uo, f, faces, b, omega, 1, stream, nullptr, false);
+        if (rc != MGP_ERR_ARG) return rc;
+    }
     MarchArgs<T> A;
     A.ui = view_of<T>(*ui);
     A.uo = view_of<T>(*uo);
@@ -2466,6 +2339,10 @@ int64_t g_sweep2_prolong = 2;  // the cycles add the prolongation inside the fir
 template <class T>
 int march_sweep2(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_array* f, const mgp_faces* faces,
                  const int64_t b[6], double omega, void* stream, const mgp_array* coarse, bool zero_in) {
+    if (g_sweep2_rows == 0 && g_sweep2_pack == 3) {
+        const int rc = tile_sweep<T>(mode, ui, uo, f, faces, b, omega, 2, stream, coarse, zero_in);
+        if (rc != MGP_ERR_ARG) return rc;
+    }
     MarchArgs<T> A;
     A.ui = view_of<T>(*ui);
     A.uo = view_of<T>(*uo);

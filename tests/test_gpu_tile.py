@@ -1,0 +1,70 @@
+"""The workgroup-tile passes (mgp_tile.hip) against the wave marches, bit for
+bit: one sweep, two sweeps, two sweeps of u + P(coarse) and of zero, at the
+sizes where tiles, remainders and chunks begin and end."""
+import ctypes
+import zlib
+
+import numpy as np
+import pytest
+
+import mgp
+
+from test_gpu_parity import random_level, shape_slices, tuned
+
+pytestmark = pytest.mark.gpu
+
+# tiles are 32 (FP64) or 64 (FP32) rows x 128 columns, two columns per lane;
+# rings of 2 (one sweep) or 4 (two sweeps) inside the box
+SHAPES = [((3, 3, 3), "NNNNNN"), ((5, 33, 17), "DDDDDD"), ((9, 32, 128), "NNDDNN"), ((8, 34, 130), "DDDDDD"),
+          ((11, 35, 131), "DNNDND"), ((7, 56, 129), "NDDNDN"), ((13, 57, 249), "NNNNDD"), ((6, 58, 248), "NNNNNN"),
+          ((9, 90, 251), "DDNNDD"), ((21, 31, 370), "NNDDNN"), ((40, 67, 61), "NNNNND"), ((17, 121, 127), "DNDNND"),
+          ((300, 9, 7), "NNNNDD"), ((65, 129, 65), "NNNNDD")]
+
+
+def level(shape, bc, mode, sfx, what):
+    dtype = np.float64 if sfx == "f64" else np.float32
+    lv = random_level(shape, bc, mode, dtype, (shape, bc, mode, what))
+    if lv is None:
+        pytest.skip("reference colouring is not a checkerboard for this halo layout")
+    return (dtype,) + lv
+
+
+def run(name, mode, u0, halo, shape, dtype, f, F, box, extra=(), zero=False):
+    """The call into a buffer that starts with other values, and its input after it."""
+    a = mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0)
+    b = mgp.DeviceArray(shape, halo, dtype=dtype).upload(np.random.default_rng(7).standard_normal(u0.shape))
+    first = [] if zero else [a.ref()]
+    mgp.call(name, mode, *first, b.ref(), f.ref(), ctypes.byref(F), mgp.box(box), 0.93, *extra, None)
+    return b.download(), a.download()
+
+
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("mode", [mgp.REFERENCE, mgp.CONSISTENT])
+@pytest.mark.parametrize("shape,bc", SHAPES, ids=["%dx%dx%d_%s" % (s + (b,)) for s, b in SHAPES])
+def test_tile_sweeps_equal_wave_marches(shape, bc, mode, sfx):
+    dtype, halo, u0, f, faces, F, box = level(shape, bc, mode, sfx, "tile")
+    rows = 12 if sfx == "f64" else 16
+    for name, keys in (("mgp_rbgs_sweep_", {"sweep__rows": rows}), ("mgp_rbgs_sweep2_", {"sweep2__rows": 16})):
+        with tuned(**keys):
+            want, _ = run(name + sfx, mode, u0, halo, shape, dtype, f, F, box)
+        got, after = run(name + sfx, mode, u0, halo, shape, dtype, f, F, box)
+        np.testing.assert_array_equal(got, want)
+        np.testing.assert_array_equal(after, u0.astype(dtype))
+
+
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("shape,bc", SHAPES, ids=["%dx%dx%d_%s" % (s + (b,)) for s, b in SHAPES])
+def test_tile_correction_and_zero_equal_wave_marches(shape, bc, sfx):
+    fine = tuple(v | 1 for v in shape)
+    dtype, halo, u0, f, faces, F, box = level(fine, bc, mgp.CONSISTENT, sfx, "tile correction")
+    cs = tuple((v - 1) // 2 + 1 for v in fine)
+    rng = np.random.default_rng(zlib.crc32(repr((shape, bc)).encode()))
+    coarse = mgp.DeviceArray(cs, halo, dtype=dtype)
+    coarse.upload(rng.standard_normal(coarse.pshape))
+    for name, extra, zero in (("mgp_rbgs_sweep2_prolong_", (coarse.ref(),), False),
+                              ("mgp_rbgs_sweep2_from_zero_", (), True)):
+        with tuned(sweep2__rows=16):
+            want, _ = run(name + sfx, mgp.CONSISTENT, u0, halo, fine, dtype, f, F, box, extra, zero)
+        got, _ = run(name + sfx, mgp.CONSISTENT, u0, halo, fine, dtype, f, F, box, extra, zero)
+        inner = shape_slices(fine, halo)
+        np.testing.assert_array_equal(got[inner], want[inner])
