@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "mgp.h"
 #include "mgp_device.h"
@@ -194,113 +195,115 @@ __global__ void k_gs_half(View<T> u, View<T> f, Box bx, int64_t zc, T one_omega,
 }
 
 // nsweeps one-pass red-black sweeps of a level that fits in one workgroup's
-// LDS, in one launch: the padded u (halos included) and f are staged in LDS;
-// each sweep is ghost refresh, red half-sweep, ghost refresh, black
-// half-sweep (include/relaxation.h:25-90), with barriers between, exactly
-// what the per-sweep kernels compute; the box points are written to uo at
-// the end.  Latency, not bandwidth, bounds the coarsest levels, and one
-// launch replaces 2 nsweeps of them.  S is the arrays' storage type, T the
-// arithmetic (and LDS) type: S = float with T = double is the FP64 solve of
-// an FP32 coarsest level (values widen exactly on load, round once on store).
-template <class S, class T, int MODE>
+// LDS, in one launch: what the per-sweep kernels compute (ghost refresh, red
+// half-sweep, ghost refresh, black half-sweep, include/relaxation.h:25-90).
+// Latency bounds the coarsest levels, so a half-sweep is one LDS round trip and
+// one barrier: a thread owns MP red and MP black points, whose value, right-hand
+// side and Neumann terms stay in its registers; u (and only u) is in LDS, the
+// points of either colour in an array of their own, so that a half-sweep's
+// neighbours are at fixed offsets in the other array and consecutive lanes read
+// consecutive words; a Neumann ghost, sign*2h*g + mirror (include/neumann.h:
+// 112-130), is formed where its neighbour is updated, the mirror being the
+// neighbour on the other side of that point.  Padding the shape with its ghost
+// layer to odd lengths makes the parity of the linear index the colour.
+// 32 sweeps of 17 x 17 x 9 with Neumann x and y faces, FP64: 31 us, against 73
+// us with ghosts refreshed in LDS, two barriers per half-sweep and every point
+// visited for either colour.  S is the arrays' storage type, T the arithmetic (and LDS)
+// type: S = float with T = double is the FP64 solve of an FP32 coarsest level
+// (values widen exactly on load, round once on store).
+template <class S, class T, int MODE, int MP>
 __global__ void __launch_bounds__(1024) k_rbgs_lds(View<S> ui, View<S> uo, View<S> f, Faces<S> F, Box bx,
                                                     int64_t nsweeps, T one_omega, T omega_sixth, T hsq, T two_h,
                                                     int64_t lin0) {
-    constexpr int MAXP = 8;  // box points per thread: <= 8192 / 1024 for any level that fits
     extern __shared__ unsigned char lds_raw[];
     T* su = reinterpret_cast<T*>(lds_raw);
-    // sizes below fit 32-bit indices (the level fits in 64 KiB)
+    // sizes below fit 32-bit indices (the level fits in LDS)
     const int n0 = (int)ui.n0, n1 = (int)ui.n1, n2 = (int)ui.n2;
-    // LDS layout: the shape with one ghost layer on every side, then f over
-    // the shape.  Ghost cells are written by the refresh before every
-    // half-sweep (Neumann faces) or never read (Dirichlet faces: the box
-    // stops one short of them), so only the shape is staged.
-    const int q2 = n2 + 2, q1 = n1 + 2;
-    const int P = (n0 + 2) * q1 * q2;
-    T* sf = su + P;
+    const int q2 = (n2 + 2) | 1, q1 = (n1 + 2) | 1;
+    const int half = ((n0 + 2) * q1 * q2 + 1) / 2;
     auto L = [&](int i, int j, int k) { return ((i + 1) * q1 + (j + 1)) * q2 + (k + 1); };
+    auto at = [&](int c) -> T& { return su[(c & 1) * half + (c >> 1)]; };
     const int tid = threadIdx.x, nt = blockDim.x;
-    for (int t = tid; t < P; t += nt) su[t] = (T)0;
-    __syncthreads();
     for (int t = tid; t < n0 * n1 * n2; t += nt) {
         const int i = t / (n1 * n2), j = (t / n2) % n1, k = t % n2;
-        su[L(i, j, k)] = (T)ui.at(i, j, k);
-        sf[t] = (T)f.at(i, j, k);
+        at(L(i, j, k)) = (T)ui.at(i, j, k);
     }
-    // this thread's box points: LDS index, f index, colour
+    // this thread's points: the m-th red (X = 0) and black (X = 1) one is
+    // number 2 (tid + m nt) or the one after it in the box, its rows and
+    // planes padded to odd lengths
     const int bn0 = (int)(bx.x1 - bx.x0), bn1 = (int)(bx.y1 - bx.y0), bn2 = (int)(bx.z1 - bx.z0);
-    const int nbox = bn0 * bn1 * bn2;
-    int pc[MAXP], pf[MAXP], pcol[MAXP];
+    const int e1 = bn1 | 1, e2 = bn2 | 1;
+    const int r0 = (int)((bx.x0 + bx.y0 + bx.z0 + (MODE == MGP_MODE_REFERENCE ? lin0 : 0)) & 1);
+    int pos[2][MP], ghost[2][MP];  // index in the colour's array (-1: none); faces whose ghost the point sees
+    T val[2][MP], rhs[2][MP], gv[2][MP][3];
+    auto point = [&](int X, int m, int& i, int& j, int& k) {
+        const int t = 2 * (tid + m * nt) + (X ^ r0);
+        i = (int)bx.x0 + t / (e1 * e2), j = (t / e2) % e1, k = t % e2;
+        const bool in = i < (int)bx.x1 && j < bn1 && k < bn2;
+        j += (int)bx.y0, k += (int)bx.z0;
+        return in;
+    };
 #pragma unroll
-    for (int m = 0; m < MAXP; m++) {
-        const int t = tid + m * nt;
-        pc[m] = -1;
-        pf[m] = 0;
-        pcol[m] = 2;
-        if (t < nbox) {
-            const int i = (int)bx.x0 + t / (bn1 * bn2), j = (int)bx.y0 + (t / bn2) % bn1, k = (int)bx.z0 + t % bn2;
-            pc[m] = L(i, j, k);
-            pf[m] = (i * n1 + j) * n2 + k;
-            pcol[m] = colour_of<MODE>(lin0, ui.s0, ui.s1, i, j, k);
-        }
-    }
-    const int s1l = q2, s0l = q1 * q2;
-    // Neumann ghosts: sign*2h*g + mirror (include/neumann.h:112-130).  Each
-    // thread owns at most one ghost cell per face (faces of a level this
-    // kernel takes have at most blockDim cells): its LDS index, the mirror's
-    // offset and the constant sign*2h*g are formed once, not per half-sweep.
-    int gc[6], gd[6];
-    T gv[6];
+    for (int X = 0; X < 2; X++)
 #pragma unroll
-    for (int q = 0; q < 6; q++) {
-        gc[q] = -1;
-        gd[q] = 0;
-        gv[q] = (T)0;
-        if (!F.neumann[q]) continue;
-        const int a0 = (q == MGP_EAST || q == MGP_WEST) ? 1 : n0;
-        const int a1 = (q == MGP_NORTH || q == MGP_SOUTH) ? 1 : n1;
-        const int a2 = (q == MGP_TOP || q == MGP_BOTTOM) ? 1 : n2;
-        const int t = tid;
-        if (t >= a0 * a1 * a2) continue;
-        const int i = t / (a1 * a2), j = (t / a2) % a1, k = t % a2;
-        int gi = i, gj = j, gk = k, d = 0;
-        T sign = (T)1.0;
-        switch (q) {
-        case MGP_EAST: gi = n0; d = -2 * s0l; break;
-        case MGP_WEST: gi = -1; d = 2 * s0l; sign = (T)-1.0; break;
-        case MGP_NORTH: gj = n1; d = -2 * s1l; break;
-        case MGP_SOUTH: gj = -1; d = 2 * s1l; sign = (T)-1.0; break;
-        case MGP_TOP: gk = n2; d = -2; break;
-        default: gk = -1; d = 2; sign = (T)-1.0; break;
+        for (int m = 0; m < MP; m++) {
+            int i, j, k;
+            pos[X][m] = -1, ghost[X][m] = 0;
+            val[X][m] = rhs[X][m] = gv[X][m][0] = gv[X][m][1] = gv[X][m][2] = (T)0;
+            if (!point(X, m, i, j, k)) continue;
+            pos[X][m] = L(i, j, k) >> 1;
+            val[X][m] = (T)ui.at(i, j, k);
+            rhs[X][m] = (T)f.at(i, j, k);
+            auto see = [&](int face, int axis, T sign, int cell) {
+                ghost[X][m] |= 1 << face;
+                gv[X][m][axis] = sign * two_h * (T)F.g[face][cell];
+            };
+            if (i == 0 && F.neumann[MGP_WEST]) see(MGP_WEST, 0, (T)-1.0, j * n2 + k);
+            else if (i == n0 - 1 && F.neumann[MGP_EAST]) see(MGP_EAST, 0, (T)1.0, j * n2 + k);
+            if (j == 0 && F.neumann[MGP_SOUTH]) see(MGP_SOUTH, 1, (T)-1.0, i * n2 + k);
+            else if (j == n1 - 1 && F.neumann[MGP_NORTH]) see(MGP_NORTH, 1, (T)1.0, i * n2 + k);
+            if (k == 0 && F.neumann[MGP_BOTTOM]) see(MGP_BOTTOM, 2, (T)-1.0, i * n1 + j);
+            else if (k == n2 - 1 && F.neumann[MGP_TOP]) see(MGP_TOP, 2, (T)1.0, i * n1 + j);
         }
-        gc[q] = L(gi, gj, gk);
-        gd[q] = d;
-        gv[q] = sign * two_h * (T)F.g[q][t];
-    }
     __syncthreads();
-    for (int64_t s = 0; s < nsweeps; s++) {
-        for (int colour = 0; colour < 2; colour++) {
+    // parity of a colour's linear indices: (i + 1) + (j + 1) + (k + 1) even or odd
+    const int red = (MODE == MGP_MODE_REFERENCE ? (int)(lin0 & 1) : 0) ^ 1;
+    auto half_sweep = [&](auto Xc) {
+        constexpr int X = decltype(Xc)::value;
+        const int pc = red ^ X;  // index parity of the points updated
+        T* own = su + pc * half;
+        const T* nb = su + (pc ^ 1) * half;
+        auto off = [&](int o) { return (o + pc) >> 1; };
 #pragma unroll
-            for (int q = 0; q < 6; q++)
-                if (gc[q] >= 0) su[gc[q]] = gv[q] + su[gc[q] + gd[q]];
-            __syncthreads();
-#pragma unroll
-            for (int m = 0; m < MAXP; m++) {
-                if (pcol[m] != colour) continue;
-                const int c = pc[m];
-                su[c] = relax_point<T, MODE>(su[c], su[c - s0l], su[c + s0l], su[c - s1l], su[c + s1l], su[c - 1],
-                                             su[c + 1], sf[pf[m]], one_omega, omega_sixth, hsq);
-            }
-            __syncthreads();
+        for (int m = 0; m < MP; m++) {
+            if (pos[X][m] < 0) continue;
+            const T* c = nb + pos[X][m];
+            T vW = c[off(-q1 * q2)], vE = c[off(q1 * q2)], vS = c[off(-q2)], vN = c[off(q2)], vB = c[off(-1)],
+              vT = c[off(1)];
+            const int g = ghost[X][m];
+            vW = g & (1 << MGP_WEST) ? gv[X][m][0] + vE : vW;
+            vE = g & (1 << MGP_EAST) ? gv[X][m][0] + vW : vE;
+            vS = g & (1 << MGP_SOUTH) ? gv[X][m][1] + vN : vS;
+            vN = g & (1 << MGP_NORTH) ? gv[X][m][1] + vS : vN;
+            vB = g & (1 << MGP_BOTTOM) ? gv[X][m][2] + vT : vB;
+            vT = g & (1 << MGP_TOP) ? gv[X][m][2] + vB : vT;
+            val[X][m] = relax_point<T, MODE>(val[X][m], vW, vE, vS, vN, vB, vT, rhs[X][m], one_omega, omega_sixth,
+                                             hsq);
+            own[pos[X][m]] = val[X][m];
         }
+        __syncthreads();
+    };
+    for (int64_t s = 0; s < nsweeps; s++) {
+        half_sweep(std::integral_constant<int, 0>{});
+        half_sweep(std::integral_constant<int, 1>{});
     }
 #pragma unroll
-    for (int m = 0; m < MAXP; m++) {
-        if (pc[m] < 0) continue;
-        const int t = tid + m * nt;
-        const int i = (int)bx.x0 + t / (bn1 * bn2), j = (int)bx.y0 + (t / bn2) % bn1, k = (int)bx.z0 + t % bn2;
-        uo.at(i, j, k) = (S)su[pc[m]];
-    }
+    for (int X = 0; X < 2; X++)
+#pragma unroll
+        for (int m = 0; m < MP; m++) {
+            int i, j, k;
+            if (point(X, m, i, j, k)) uo.at(i, j, k) = (S)val[X][m];
+        }
     // out of place: the shape points outside the box as loaded, so u_out is a
     // complete image of the in-place result (the boundary points' own history,
     // signs of zero included, follows whichever buffer ends up current)
@@ -308,7 +311,7 @@ __global__ void __launch_bounds__(1024) k_rbgs_lds(View<S> ui, View<S> uo, View<
         for (int t = tid; t < n0 * n1 * n2; t += nt) {
             const int i = t / (n1 * n2), j = (t / n2) % n1, k = t % n2;
             if (i >= bx.x0 && i < bx.x1 && j >= bx.y0 && j < bx.y1 && k >= bx.z0 && k < bx.z1) continue;
-            uo.at(i, j, k) = (S)su[L(i, j, k)];
+            uo.at(i, j, k) = (S)at(L(i, j, k));
         }
     }
 }
@@ -1079,12 +1082,28 @@ static int rbgs_sweeps(int mode, const mgp_array* ui, const mgp_array* uo, const
     const T two_h = (T)(2.0 * faces->h);  // include/neumann.h:108, in the arithmetic type
     const View<S> vi = view_of<S>(*ui);
     const hipStream_t s = (hipStream_t)stream;
-    if (mode == MGP_MODE_REFERENCE)
-        hipLaunchKernelGGL((k_rbgs_lds<S, T, MGP_MODE_REFERENCE>), dim3(1), dim3(1024), lds, s, vi, view_of<S>(*uo),
-                           view_of<S>(*f), F, bx, nsweeps, c.one_omega, c.omega_sixth, c.hsq, two_h, lin0_of(ui));
-    else
-        hipLaunchKernelGGL((k_rbgs_lds<S, T, MGP_MODE_CONSISTENT>), dim3(1), dim3(1024), lds, s, vi, view_of<S>(*uo),
-                           view_of<S>(*f), F, bx, nsweeps, c.one_omega, c.omega_sixth, c.hsq, two_h, lin0_of(ui));
+    // red (and black) points, the box's rows and planes padded to odd lengths:
+    // at most 2048 in FP64 and 4096 in FP32, by the limit on the level above
+    const int64_t pts = ((b[1] - b[0]) * ((b[3] - b[2]) | 1) * ((b[5] - b[4]) | 1) + 1) / 2;
+    const dim3 blk((unsigned)std::min<int64_t>(1024, (pts + 63) / 64 * 64));
+    const size_t bytes = ((size_t)(n0 + 2) * ((n1 + 2) | 1) * ((n2 + 2) | 1) + 1) / 2 * 2 * sizeof(T);
+#define MGP_LDS_LAUNCH(M, PP)                                                                                        \
+    hipLaunchKernelGGL((k_rbgs_lds<S, T, M, PP>), dim3(1), blk, bytes, s, vi, view_of<S>(*uo), view_of<S>(*f), F, bx, \
+                       nsweeps, c.one_omega, c.omega_sixth, c.hsq, two_h, lin0_of(ui))
+    const bool ref = mode == MGP_MODE_REFERENCE;
+    if (pts <= 1024) {
+        if (ref) MGP_LDS_LAUNCH(MGP_MODE_REFERENCE, 1);
+        else MGP_LDS_LAUNCH(MGP_MODE_CONSISTENT, 1);
+    } else if (pts <= 2048) {
+        if (ref) MGP_LDS_LAUNCH(MGP_MODE_REFERENCE, 2);
+        else MGP_LDS_LAUNCH(MGP_MODE_CONSISTENT, 2);
+    } else if (pts <= 4096) {
+        if (ref) MGP_LDS_LAUNCH(MGP_MODE_REFERENCE, 4);
+        else MGP_LDS_LAUNCH(MGP_MODE_CONSISTENT, 4);
+    } else {
+        return MGP_ERR_ARG;
+    }
+#undef MGP_LDS_LAUNCH
     return launch_status();
 }
 

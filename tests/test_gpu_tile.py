@@ -68,3 +68,21 @@ def test_tile_correction_and_zero_equal_wave_marches(shape, bc, sfx):
         got, _ = run(name + sfx, mgp.CONSISTENT, u0, halo, fine, dtype, f, F, box, extra, zero)
         inner = shape_slices(fine, halo)
         np.testing.assert_array_equal(got[inner], want[inner])
+
+
+# one workgroup, points per thread and colour: 2 (FP64 and FP32) and 4 (FP32),
+# odd and even box lengths
+@pytest.mark.parametrize("sfx,shape,bc", [("f64", (15, 15, 14), "NNNNNN"), ("f64", (15, 15, 14), "DNNDND"),
+                                          ("f32", (19, 19, 19), "DDDDDD"), ("f32", (18, 20, 19), "NDDNDN"),
+                                          ("f64", (40, 2, 3), "NNDDDD"), ("f32", (16, 14, 15), "NNNNNN")])
+@pytest.mark.parametrize("mode", [mgp.REFERENCE, mgp.CONSISTENT])
+def test_lds_sweeps_with_several_points_per_thread(mode, sfx, shape, bc):
+    dtype, halo, u0, f, faces, F, box = level(shape, bc, mode, sfx, "lds")
+    a = mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0)
+    b = mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0)
+    c = mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0)
+    mgp.call("mgp_rbgs_sweeps_" + sfx, mode, a.ref(), c.ref(), f.ref(), ctypes.byref(F), mgp.box(box), 0.93, 3, None)
+    for _ in range(3):
+        mgp.call("mgp_rbgs_sweep_" + sfx, mode, a.ref(), b.ref(), f.ref(), ctypes.byref(F), mgp.box(box), 0.93, None)
+        a, b = b, a
+    np.testing.assert_array_equal(c.download(), a.download())
