@@ -603,10 +603,15 @@ int mgp_cycle_noalloc_f64(const char* cycle, const mgp_array* u, const mgp_array
  * loads in flight per wave, kernel 2, default 1), "sweep.pair" (1: the
  * GaussSeidel smoother runs its sweeps in pairs through mgp_rbgs_sweep2_*,
  * default; 0: one pass per sweep), "sweep.pair_min_points" (levels with fewer
- * points run one pass per sweep; default 2^20), "sweep.tile" (workgroup tiles
+ * points run one pass per sweep; default 0), "sweep.tile" (workgroup tiles
  * with values in registers, bit 0 for mgp_rbgs_sweep_*, bit 1 for the
  * two-sweep passes; used while "sweep.kernel", "sweep.rows" and "sweep.depth",
  * or "sweep2.rows" and "sweep2.pack", have their defaults; default 3),
+ * "sweep2.blocks" (two sweeps of a level that this many blocks of 16 x 12 or
+ * 16 x 64 points cover run as blocks, one workgroup each, under the same keys;
+ * default 256, 0: none), "residual_fw.block_points" (fine levels of at most this many
+ * points take the fused residual and full-weighting restriction in blocks
+ * while "residual_fw.rows" and "residual_fw.depth" are 0; default 2^21),
  * "sweep.small_points" and
  * "sweep.small_min_chunk" (levels with fewer points than the first use the
  * second as their shortest x march; defaults 2^18 and 1), "sweep2.rows"

@@ -28,6 +28,17 @@ template <class T>
 int tile_sweep(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_array* f, const mgp_faces* faces,
                const int64_t box[6], double omega, int sweeps, void* stream, const mgp_array* coarse, bool zero_in);
 extern int64_t g_tile;
+// two sweeps of a small level through blocks (mgp_block.hip)
+template <class T>
+int block_sweep(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_array* f, const mgp_faces* faces,
+                const int64_t box[6], double omega, void* stream, const mgp_array* coarse, bool zero_in);
+extern int64_t g_block_count;  // most blocks of a launch
+// residual + full weighting through blocks (mgp_descend.hip; arguments as
+// march_residual_fw)
+template <class T>
+int block_residual_fw(const mgp_array* u, const mgp_array* f, const mgp_array* r, const mgp_array* cf,
+                      const int64_t b[6], double h, void* stream);
+extern int64_t g_fw_block_points;  // largest fine level they take
 extern int64_t g_sweep_pair;
 extern int64_t g_sweep2_rows;
 extern int64_t g_sweep2_prolong;

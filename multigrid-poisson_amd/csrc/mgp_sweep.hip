@@ -62,11 +62,10 @@ static inline int64_t target_wgs(int64_t own) { return own > 0 ? own : g_sweep_t
 int64_t g_small_points = 1 << 18;
 int64_t g_small_min_chunk = 1;
 // the Gauss-Seidel smoother pairs its sweeps (mgp_rbgs_sweep2_*) on levels of
-// at least this many points (workgroup tiles, FP64: 257 x 257 x 129 pair 84 us,
-// two sweeps 104 us; 129 x 129 x 65 pair 36 us, two sweeps 32 us, but with the
-// correction inside 44 us against 46 us and one launch less; 65 x 65 x 33 pair
-// 24 us, two sweeps 21 us)
-int64_t g_pair_min_points = 1 << 20;
+// at least this many points: every level.  FP64, Neumann x and y faces, pair /
+// two sweeps: 257 x 257 x 129 84 / 104 us, 129 x 129 x 65 39 / 35 us (with the
+// correction inside 47 / 47 us and one launch less), 65 x 65 x 33 15 / 22 us
+int64_t g_pair_min_points = 0;
 extern int64_t g_sweep_min_chunk;
 static inline int64_t min_chunk_for(int64_t points) {
     return points < g_small_points ? g_small_min_chunk : g_sweep_min_chunk;
@@ -2253,6 +2252,10 @@ int march_residual_fw(const mgp_array* u, const mgp_array* f, const mgp_array* r
             return MGP_ERR_ARG;
     for (int q = 0; q < 6; q++)
         if (u->halo[q] != f->halo[q] || u->halo[q] != r->halo[q]) return MGP_ERR_ARG;
+    if (g_fw_rows == 0 && g_fw_depth == 0) {
+        const int rc = block_residual_fw<T>(u, f, r, cf, b, h, stream);
+        if (rc != MGP_ERR_ARG) return rc;
+    }
     RFArgs<T> A;
     A.u = view_of<T>(*u);
     A.f = view_of<T>(*f);
@@ -2340,7 +2343,8 @@ template <class T>
 int march_sweep2(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_array* f, const mgp_faces* faces,
                  const int64_t b[6], double omega, void* stream, const mgp_array* coarse, bool zero_in) {
     if (g_sweep2_rows == 0 && g_sweep2_pack == 3) {
-        const int rc = tile_sweep<T>(mode, ui, uo, f, faces, b, omega, 2, stream, coarse, zero_in);
+        int rc = block_sweep<T>(mode, ui, uo, f, faces, b, omega, stream, coarse, zero_in);
+        if (rc == MGP_ERR_ARG) rc = tile_sweep<T>(mode, ui, uo, f, faces, b, omega, 2, stream, coarse, zero_in);
         if (rc != MGP_ERR_ARG) return rc;
     }
     MarchArgs<T> A;

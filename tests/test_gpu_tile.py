@@ -1,5 +1,5 @@
-"""The workgroup-tile passes (mgp_tile.hip) against the wave marches, bit for
-bit: one sweep, two sweeps, two sweeps of u + P(coarse) and of zero, at the
+"""The workgroup-tile passes (mgp_tile.hip) and the block passes of small levels
+(mgp_block.hip, mgp_descend.hip) against the wave marches, bit for bit: one sweep, two sweeps, two sweeps of u + P(coarse) and of zero, at the
 sizes where tiles, remainders and chunks begin and end."""
 import ctypes
 import zlib
@@ -13,7 +13,9 @@ from test_gpu_parity import random_level, shape_slices, tuned
 
 pytestmark = pytest.mark.gpu
 
-# tiles are 32 (FP64) or 64 (FP32) rows x 128 columns, two columns per lane;
+# most blocks of a launch: none (then tiles), or every level here
+PATHS = {"tile": 0, "block": 1 << 20}
+# blocks are 16 planes x 12 (FP64) or 16 (FP32) rows x 64 columns.  Tiles are 32 (FP64) or 64 (FP32) rows x 128 columns, two columns per lane;
 # rings of 2 (one sweep) or 4 (two sweeps) inside the box
 SHAPES = [((3, 3, 3), "NNNNNN"), ((5, 33, 17), "DDDDDD"), ((9, 32, 128), "NNDDNN"), ((8, 34, 130), "DDDDDD"),
           ((11, 35, 131), "DNNDND"), ((7, 56, 129), "NDDNDN"), ((13, 57, 249), "NNNNDD"), ((6, 58, 248), "NNNNNN"),
@@ -38,23 +40,26 @@ def run(name, mode, u0, halo, shape, dtype, f, F, box, extra=(), zero=False):
     return b.download(), a.download()
 
 
+@pytest.mark.parametrize("path", list(PATHS))
 @pytest.mark.parametrize("sfx", ["f64", "f32"])
 @pytest.mark.parametrize("mode", [mgp.REFERENCE, mgp.CONSISTENT])
 @pytest.mark.parametrize("shape,bc", SHAPES, ids=["%dx%dx%d_%s" % (s + (b,)) for s, b in SHAPES])
-def test_tile_sweeps_equal_wave_marches(shape, bc, mode, sfx):
+def test_tile_sweeps_equal_wave_marches(shape, bc, mode, sfx, path):
     dtype, halo, u0, f, faces, F, box = level(shape, bc, mode, sfx, "tile")
     rows = 12 if sfx == "f64" else 16
     for name, keys in (("mgp_rbgs_sweep_", {"sweep__rows": rows}), ("mgp_rbgs_sweep2_", {"sweep2__rows": 16})):
         with tuned(**keys):
             want, _ = run(name + sfx, mode, u0, halo, shape, dtype, f, F, box)
-        got, after = run(name + sfx, mode, u0, halo, shape, dtype, f, F, box)
+        with tuned(sweep2__blocks=PATHS[path]):
+            got, after = run(name + sfx, mode, u0, halo, shape, dtype, f, F, box)
         np.testing.assert_array_equal(got, want)
         np.testing.assert_array_equal(after, u0.astype(dtype))
 
 
+@pytest.mark.parametrize("path", list(PATHS))
 @pytest.mark.parametrize("sfx", ["f64", "f32"])
 @pytest.mark.parametrize("shape,bc", SHAPES, ids=["%dx%dx%d_%s" % (s + (b,)) for s, b in SHAPES])
-def test_tile_correction_and_zero_equal_wave_marches(shape, bc, sfx):
+def test_tile_correction_and_zero_equal_wave_marches(shape, bc, sfx, path):
     fine = tuple(v | 1 for v in shape)
     dtype, halo, u0, f, faces, F, box = level(fine, bc, mgp.CONSISTENT, sfx, "tile correction")
     cs = tuple((v - 1) // 2 + 1 for v in fine)
@@ -65,9 +70,29 @@ def test_tile_correction_and_zero_equal_wave_marches(shape, bc, sfx):
                               ("mgp_rbgs_sweep2_from_zero_", (), True)):
         with tuned(sweep2__rows=16):
             want, _ = run(name + sfx, mgp.CONSISTENT, u0, halo, fine, dtype, f, F, box, extra, zero)
-        got, _ = run(name + sfx, mgp.CONSISTENT, u0, halo, fine, dtype, f, F, box, extra, zero)
+        with tuned(sweep2__blocks=PATHS[path]):
+            got, _ = run(name + sfx, mgp.CONSISTENT, u0, halo, fine, dtype, f, F, box, extra, zero)
         inner = shape_slices(fine, halo)
         np.testing.assert_array_equal(got[inner], want[inner])
+
+
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("shape,bc", SHAPES, ids=["%dx%dx%d_%s" % (s + (b,)) for s, b in SHAPES])
+def test_block_descent_equals_wave_march(shape, bc, sfx):
+    """mgp_residual_restrict_fw through blocks, r as stored outside the box."""
+    dtype, halo, u0, f, faces, F, box = level(shape, bc, mgp.CONSISTENT, sfx, "descent")
+    cs = tuple((v - 1) // 2 + 1 for v in shape)
+    u = mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0)
+    r = mgp.DeviceArray(shape, halo, dtype=dtype).upload(np.random.default_rng(3).standard_normal(u0.shape))
+    got = []
+    for rows, points in ((6, 0), (0, 1 << 24)):
+        c = mgp.DeviceArray(cs, halo, dtype=dtype)
+        c.upload(np.random.default_rng(5).standard_normal(c.pshape))
+        with tuned(residual_fw__rows=rows, residual_fw__block_points=points):
+            mgp.call("mgp_residual_restrict_fw_" + sfx, mgp.CONSISTENT, u.ref(), f.ref(), r.ref(), c.ref(),
+                     mgp.box(box), F.h, None)
+        got.append(c.download())
+    np.testing.assert_array_equal(got[1], got[0])
 
 
 # one workgroup, points per thread and colour: 2 (FP64 and FP32) and 4 (FP32),
