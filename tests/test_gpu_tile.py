@@ -76,16 +76,18 @@ def test_tile_correction_and_zero_equal_wave_marches(shape, bc, sfx, path):
         np.testing.assert_array_equal(got[inner], want[inner])
 
 
+@pytest.mark.parametrize("points", [0, 1 << 24], ids=["march", "block"])
 @pytest.mark.parametrize("sfx", ["f64", "f32"])
 @pytest.mark.parametrize("shape,bc", SHAPES, ids=["%dx%dx%d_%s" % (s + (b,)) for s, b in SHAPES])
-def test_block_descent_equals_wave_march(shape, bc, sfx):
-    """mgp_residual_restrict_fw through blocks, r as stored outside the box."""
+def test_descents_equal_wave_march(shape, bc, sfx, points):
+    """mgp_residual_restrict_fw through blocks and through the march with
+    running sums, r as stored outside the box."""
     dtype, halo, u0, f, faces, F, box = level(shape, bc, mgp.CONSISTENT, sfx, "descent")
     cs = tuple((v - 1) // 2 + 1 for v in shape)
     u = mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0)
     r = mgp.DeviceArray(shape, halo, dtype=dtype).upload(np.random.default_rng(3).standard_normal(u0.shape))
     got = []
-    for rows, points in ((6, 0), (0, 1 << 24)):
+    for rows in (6, 0):
         c = mgp.DeviceArray(cs, halo, dtype=dtype)
         c.upload(np.random.default_rng(5).standard_normal(c.pshape))
         with tuned(residual_fw__rows=rows, residual_fw__block_points=points):
