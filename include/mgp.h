@@ -607,9 +607,9 @@ int mgp_cycle_noalloc_f64(const char* cycle, const mgp_array* u, const mgp_array
  * with values in registers, bit 0 for mgp_rbgs_sweep_*, bit 1 for the
  * two-sweep passes; used while "sweep.kernel", "sweep.rows" and "sweep.depth",
  * or "sweep2.rows" and "sweep2.pack", have their defaults; default 3),
- * "sweep2.blocks" (two sweeps of a level that this many blocks of 16 x 12 or
- * 16 x 64 points cover run as blocks, one workgroup each, under the same keys;
- * default 256, 0: none), "residual_fw.block_points" (fine levels of at most this many
+ * "sweep2.blocks" (two sweeps of a level that this many blocks of 16 planes x 12
+ * (FP64) or 16 (FP32) rows x 64 columns cover run as blocks, one workgroup each,
+ * under the same keys; default 256, 0: none), "residual_fw.block_points" (fine levels of at most this many
  * points take the fused residual and full-weighting restriction in blocks
  * while "residual_fw.rows" and "residual_fw.depth" are 0; default 2^21),
  * "sweep.small_points" and
@@ -638,6 +638,7 @@ int mgp_cycle_noalloc_f64(const char* cycle, const mgp_array* u, const mgp_array
  * and full-weighting restriction; 0 = 6, default), "residual_fw.depth" (1 or
  * 2 fine planes of loads in flight per wave; 0 = 1 for FP64 and 2 for FP32,
  * default),
+ * "jacobi.kernel" (1: per-point kernel; 2: wave tiles marching along x, default),
  * "prolong.kernel" (1: per-point kernel; 2: wave tiles marching along x for
  * mgp_prolong_add_*, default), "batch.blocks" (workgroups per launch of the
  * batched solver's work lists, default 16384).

@@ -231,7 +231,7 @@ __global__ void __launch_bounds__(1024) k_rbgs_lds(View<S> ui, View<S> uo, View<
     // this thread's points: the m-th red (X = 0) and black (X = 1) one is
     // number 2 (tid + m nt) or the one after it in the box, its rows and
     // planes padded to odd lengths
-    const int bn0 = (int)(bx.x1 - bx.x0), bn1 = (int)(bx.y1 - bx.y0), bn2 = (int)(bx.z1 - bx.z0);
+    const int bn1 = (int)(bx.y1 - bx.y0), bn2 = (int)(bx.z1 - bx.z0);
     const int e1 = bn1 | 1, e2 = bn2 | 1;
     const int r0 = (int)((bx.x0 + bx.y0 + bx.z0 + (MODE == MGP_MODE_REFERENCE ? lin0 : 0)) & 1);
     int pos[2][MP], ghost[2][MP];  // index in the colour's array (-1: none); faces whose ghost the point sees
@@ -1152,16 +1152,16 @@ static int jacobi(int mode, const mgp_array* u, const mgp_array* v, const mgp_ar
         return MGP_ERR_ARG;
     const Box bx = box_of(b);
     if (box_empty(bx)) return MGP_OK;
+    if (mode != MGP_MODE_REFERENCE && mode != MGP_MODE_CONSISTENT) return MGP_ERR_ARG;
+    if (g_jacobi_kernel == 2 && march_jacobi<T>(mode, u, v, f, b, omega, h, stream) == MGP_OK) return MGP_OK;
     const BoxGrid g = box_grid(bx);
     const RelaxConsts<T> c(omega, h);
     if (mode == MGP_MODE_REFERENCE)
         hipLaunchKernelGGL((k_jacobi<T, MGP_MODE_REFERENCE>), g.grid, g.block, 0, (hipStream_t)stream, view_of<T>(*u),
                            view_of<T>(*v), view_of<T>(*f), bx, g.zchunks, c.one_omega, c.omega_sixth, c.hsq);
-    else if (mode == MGP_MODE_CONSISTENT)
+    else
         hipLaunchKernelGGL((k_jacobi<T, MGP_MODE_CONSISTENT>), g.grid, g.block, 0, (hipStream_t)stream, view_of<T>(*u),
                            view_of<T>(*v), view_of<T>(*f), bx, g.zchunks, c.one_omega, c.omega_sixth, c.hsq);
-    else
-        return MGP_ERR_ARG;
     return launch_status();
 }
 

@@ -44,6 +44,11 @@ extern int64_t g_sweep2_rows;
 extern int64_t g_sweep2_prolong;
 extern int64_t g_sweep2_pack;
 extern int64_t g_sweep2_waves;
+// Jacobi sweep (mgp_jacobi.hip); MGP_ERR_ARG when the layout does not allow it
+template <class T>
+int march_jacobi(int mode, const mgp_array* u, const mgp_array* v, const mgp_array* f, const int64_t box[6],
+                 double omega, double h, void* stream);
+extern int64_t g_jacobi_kernel;
 // residual on a box through wave tiles (norm: max |r| over the whole shape
 // folded into *norm); MGP_ERR_ARG when the layouts do not allow it
 template <class T>

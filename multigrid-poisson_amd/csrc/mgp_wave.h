@@ -146,5 +146,30 @@ __device__ __forceinline__ void bstore(float v, __amdgpu_buffer_rsrc_t r, uint32
                                           MGP_STORE_POLICY);
 }
 
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// two adjacent values of a row (no alignment beyond the element's)
+template <class T>
+__device__ __forceinline__ void bload2(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, T& a, T& b) {
+    if constexpr (sizeof(T) == 8) {
+        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
+        a = __builtin_bit_cast(double, (u32x2){v.x, v.y});
+        b = __builtin_bit_cast(double, (u32x2){v.z, v.w});
+    } else {
+        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
+        const unsigned int x = v.x, y = v.y;  // (a bit cast of the component itself reads v.x for both)
+        a = __builtin_bit_cast(float, x);
+        b = __builtin_bit_cast(float, y);
+    }
+}
+__device__ __forceinline__ void bstore2(double a, double b, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    const u32x2 x = __builtin_bit_cast(u32x2, a), y = __builtin_bit_cast(u32x2, b);
+    __builtin_amdgcn_raw_buffer_store_b128((u32x4){x.x, x.y, y.x, y.y}, r, (int)voff, (int)soff, 0);
+}
+__device__ __forceinline__ void bstore2(float a, float b, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_buffer_store_b64(
+        (u32x2){__builtin_bit_cast(unsigned int, a), __builtin_bit_cast(unsigned int, b)}, r, (int)voff, (int)soff, 0);
+}
+
 }  // namespace
 }  // namespace mgp

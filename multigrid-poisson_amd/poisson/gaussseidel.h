@@ -74,7 +74,8 @@ public:
         int_t s = 0;
         int64_t pair = 1, pair_min = 0;
         if (mgp_tuning_get("sweep.pair", &pair) != MGP_OK) pair = 1;
-        // pairs pay on large levels only (two one-pass sweeps are faster below)
+        // (two one-pass sweeps are slower at every size: "sweep.pair_min_points"
+        // is 0 by default)
         if (mgp_tuning_get("sweep.pair_min_points", &pair_min) == MGP_OK &&
             d.u->shape[0] * d.u->shape[1] * d.u->shape[2] < pair_min)
             pair = 0;
@@ -131,9 +132,9 @@ public:
     // (mgp_rbgs_sweep2_prolong_*) where relax_level would run that pair through
     // the two-sweep pass: consistent mode, trilinear prolongation, a level of at
     // least "sweep.pair_min_points" points, "sweep2.prolong" 2 (FP64 and FP32
-    // levels, default) or 1 (FP64 levels only).  1025 x 1025 x 513: FP64 5.18 ms
-    // against 4.54 + 2.05 ms for the separate passes, FP32 2.43 against
-    // 2.30 + 1.01 ms
+    // levels, default) or 1 (FP64 levels only).  1025 x 1025 x 513: FP64 3.69 ms
+    // against 3.50 + 2.05 ms for the separate passes, FP32 1.90 against
+    // 1.79 + 1.01 ms
     void relax_level_prolonged(Domain<T>& d, Domain<T>& coarse, Prolongation<T>& prolongation, T omega,
                                int_t nsmooth) override {
         d.materialize_zero();

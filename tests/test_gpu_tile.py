@@ -1,6 +1,8 @@
-"""The workgroup-tile passes (mgp_tile.hip) and the block passes of small levels
-(mgp_block.hip, mgp_descend.hip) against the wave marches, bit for bit: one sweep, two sweeps, two sweeps of u + P(coarse) and of zero, at the
-sizes where tiles, remainders and chunks begin and end."""
+"""The workgroup-tile passes (mgp_tile.hip), the block passes of small levels
+(mgp_block.hip, mgp_descend.hip) and the Jacobi march (mgp_jacobi.hip) against
+the wave marches and the per-point kernel, bit for bit: one sweep, two sweeps,
+two sweeps of u + P(coarse) and of zero, at the sizes where tiles, remainders
+and chunks begin and end."""
 import ctypes
 import zlib
 
@@ -94,6 +96,28 @@ def test_descents_equal_wave_march(shape, bc, sfx, points):
             mgp.call("mgp_residual_restrict_fw_" + sfx, mgp.CONSISTENT, u.ref(), f.ref(), r.ref(), c.ref(),
                      mgp.box(box), F.h, None)
         got.append(c.download())
+    np.testing.assert_array_equal(got[1], got[0])
+
+
+# tiles of 16 rows x 124 columns; the three arrays with halos of their own
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("mode", [mgp.REFERENCE, mgp.CONSISTENT])
+@pytest.mark.parametrize("shape,bc", SHAPES + [((4, 17, 124), "NNNNNN"), ((3, 16, 125), "NNNNNN"),
+                                               ((5, 4, 250), "DDDDDD"), ((2, 20, 2), "NNNNNN")])
+def test_jacobi_march_equals_per_point(shape, bc, mode, sfx):
+    dtype = np.float64 if sfx == "f64" else np.float32
+    rng = np.random.default_rng(zlib.crc32(repr((shape, bc, mode, sfx)).encode()))
+    box = [v for d in range(3) for v in (0 if bc[2 * d] == "N" else 1, shape[d] - (bc[2 * d + 1] == "D"))]
+    v, f = (mgp.DeviceArray(shape, halo, dtype=dtype) for halo in ((1,) * 6, (2, 0, 1, 3, 0, 1)))
+    for a in (v, f):
+        a.upload(rng.standard_normal(a.pshape))
+    got = []
+    for kernel in (1, 2):
+        u = mgp.DeviceArray(shape, (0, 1, 0, 2, 1, 0), dtype=dtype)
+        u.upload(np.random.default_rng(7).standard_normal(u.pshape))
+        with tuned(jacobi__kernel=kernel):
+            mgp.call("mgp_jacobi_" + sfx, mode, u.ref(), v.ref(), f.ref(), mgp.box(box), 6.0 / 7.0, 1.0 / 16, None)
+        got.append(u.download())
     np.testing.assert_array_equal(got[1], got[0])
 
 
