@@ -629,9 +629,9 @@ int mgp_cycle_noalloc_f64(const char* cycle, const mgp_array* u, const mgp_array
  * residual, the fused residual + full-weighting and the prolongation marches
  * aim for; 0 = the value of
  * "sweep.target_wgs"; defaults 4096, 32768, 65536), "update_residual.target_wgs"
- * (waves of mgp_update_residual_f64_f32 and the hi + lo kernels; default 65536),
- * "update_residual.rows" (8 or 16 register rows per wave tile of the hi + lo
- * kernels, default 16), "residual.kernel" (1:
+ * (waves of mgp_update_residual_f64_f32 and the hi + lo kernels, twice as many with
+ * 8 rows; default 65536), "update_residual.rows" (8 or 16 register rows per wave
+ * tile of the hi + lo kernels, default 8), "residual.kernel" (1:
  * per-point kernels; 2: one wave per tile marching along x, default),
  * "residual.rows" (8 or 16 register rows per residual tile, default 16),
  * "residual_fw.rows" (4 or 6 coarse rows per wave tile of the fused residual

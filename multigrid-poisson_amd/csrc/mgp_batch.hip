@@ -113,6 +113,37 @@ __device__ __forceinline__ int xcd_rank() {
     return G % 8 ? b : (b % 8) * (G / 8) + b / 8;
 }
 
+// FP64 residual of one item's column k, written as the next iteration's FP32
+// right-hand side: the march of march_item (one new x-plane value per point);
+// returns max |r|
+__device__ __forceinline__ double march_residual64(const BTop& t, const View<float>& out, const BItem& item,
+                                                   int64_t k) {
+    const double* __restrict__ q = t.u.p;
+    const double* __restrict__ fp = t.f.p;
+    float* __restrict__ o = out.p;
+    const int64_t s0 = t.u.s0, s1 = t.u.s1, f0 = t.f.s0, o0 = out.s0;
+    const double inv_h2 = t.inv_h2;
+    double vmax = 0.0;
+    for (int64_t j = item.y0 + threadIdx.y; j < item.y1; j += blockDim.y) {
+        int64_t c = t.u.ix(item.x0, j, k), cf = t.f.ix(item.x0, j, k), co = out.ix(item.x0, j, k);
+        double um = q[c - s0], uc = q[c];
+        for (int64_t i = item.x0; i < item.x1; i++) {
+            const double up = q[c + s0];
+            const double sum = ((um - uc) + (up - uc)) + ((q[c - s1] - uc) + (q[c + s1] - uc)) +
+                               ((q[c - 1] - uc) + (q[c + 1] - uc));
+            const double rv = fma(-inv_h2, sum, fp[cf]);
+            o[co] = (float)rv;
+            vmax = fmax(vmax, fabs(rv));
+            um = uc;
+            uc = up;
+            c += s0;
+            cf += f0;
+            co += o0;
+        }
+    }
+    return vmax;
+}
+
 // max |.| of the FP64 residual or of f per problem: each workgroup walks a
 // contiguous run of items (the lists hold each problem's items together) and
 // keeps the running max of the problem at hand, folding it into the
@@ -143,19 +174,11 @@ __device__ __forceinline__ void batch_norms(const BArgs& a) {
         const BTop& t = a.tops[p];
         const int64_t k = item.z0 + threadIdx.x;
         const int64_t kz1 = t.u.n2;
-        if (OP == OP_RESIDUAL64 ? (k < kz1 - 1 && k >= 1) : k < kz1) {
-            for (int64_t j = item.y0 + threadIdx.y; j < item.y1; j += blockDim.y) {
-                for (int64_t i = item.x0; i < item.x1; i++) {
-                    if (OP == OP_RESIDUAL64) {
-                        const double rv = residual_point<double, MGP_MODE_CONSISTENT>(t.u, t.u.ix(i, j, k),
-                                                                                      t.f.at(i, j, k), t.hsq, t.inv_h2);
-                        a.grids[item.grid].f.at(i, j, k) = (float)rv;  // the next iteration's right-hand side
-                        vmax = fmax(vmax, fabs(rv));
-                    } else {
-                        vmax = fmax(vmax, fabs(t.f.at(i, j, k)));
-                    }
-                }
-            }
+        if (OP == OP_RESIDUAL64) {
+            if (k < kz1 - 1 && k >= 1) vmax = fmax(vmax, march_residual64(t, a.grids[item.grid].f, item, k));
+        } else if (k < kz1) {
+            for (int64_t j = item.y0 + threadIdx.y; j < item.y1; j += blockDim.y)
+                for (int64_t i = item.x0; i < item.x1; i++) vmax = fmax(vmax, fabs(t.f.at(i, j, k)));
         }
     }
     if (cur >= 0) flush();

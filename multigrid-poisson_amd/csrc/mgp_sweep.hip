@@ -50,7 +50,8 @@ int64_t g_resid_target = 4096;
 int64_t g_fw_target = 32768;
 int64_t g_prolong_target = 65536;
 // the FP64 update + residual of mixed-precision refinement: 4.59 ms with 16384
-// waves, 4.48 ms with 65536 (1025 x 1025 x 513)
+// waves, 4.48 ms with 65536 (1025 x 1025 x 513); the hi + lo kernels aim for
+// twice as many with 8 rows
 int64_t g_upd_target = 65536;
 extern int64_t g_sweep_target_wgs;
 static inline int64_t target_wgs(int64_t own) { return own > 0 ? own : g_sweep_target_wgs; }
@@ -2100,8 +2101,17 @@ int march_update_residual(int mode, const mgp_array* u, const mgp_array* un, con
     return err == hipSuccess ? MGP_OK : (int)err;
 }
 
-// rows per wave tile of the hi + lo update + residual: 8 or 16
-int64_t g_hilo_rows = 16;
+// rows per wave tile of the hi + lo update + residual: 8 or 16.  At 8 the march
+// runs two waves per SIMD instead of one, and twice as many waves share the
+// planes in flight; x chunks of 6 planes at least.  FP64 update + residual,
+// 8 rows / 16 rows: 1025 x 1025 x 513 5.60 / 6.05 ms (21.6 GB moved: 3.9 TB/s),
+// 801 x 609 x 417 2.40 / 2.65 ms, 513 x 513 x 257 757 / 762 us (774 with chunks
+// of 4 planes), 257 x 257 x 129 125 / 129 us.  Measured and left: two columns
+// per lane on 4 rows, four waves to a workgroup (6.29 ms, 2.37 ms, 803 us, 155
+// us: the ghosts of both columns spill), the same on 8 rows (5.93 ms, 2.32 ms,
+// 855 us, 172 us).
+int64_t g_hilo_rows = 8;
+constexpr int64_t HILO_MIN_CHUNK = 6;
 
 int march_hilo_residual(const mgp_array* u, const mgp_array* un, const mgp_array* lo, const mgp_array* ln,
                         const mgp_array* e, const mgp_array* f, const mgp_array* r, const mgp_array* out,
@@ -2153,8 +2163,9 @@ int march_hilo_residual(const mgp_array* u, const mgp_array* un, const mgp_array
         A.ytiles = (int)((ny + R - 1) / R);
         A.ztiles = (int)((nz + RZ - 1) / RZ);
         const int64_t tiles = (int64_t)A.ytiles * A.ztiles;
-        int64_t chunks = std::max<int64_t>(1, target_wgs(g_upd_target) / std::max<int64_t>(tiles, 1));
-        chunks = std::min<int64_t>(chunks, std::max<int64_t>(1, nx / std::max<int64_t>(min_chunk_for(box_points(b)), 1)));
+        int64_t chunks = std::max<int64_t>(1, (R == 8 ? 2 : 1) * target_wgs(g_upd_target) / std::max<int64_t>(tiles, 1));
+        const int64_t shortest = R == 8 && box_points(b) >= g_small_points ? HILO_MIN_CHUNK : min_chunk_for(box_points(b));
+        chunks = std::min<int64_t>(chunks, std::max<int64_t>(1, nx / std::max<int64_t>(shortest, 1)));
         A.xchunk = (nx + chunks - 1) / chunks;
         A.ntiles = (int)(tiles * ((nx + A.xchunk - 1) / A.xchunk));
         A.ntiles_pad = (A.ntiles + 7) / 8 * 8;
