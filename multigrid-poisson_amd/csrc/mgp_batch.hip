@@ -157,10 +157,8 @@ __device__ __forceinline__ void batch_norms(const BArgs& a) {
     double vmax = 0.0;
     auto flush = [&]() {
         vmax = wave_max64(vmax);
-        if ((threadIdx.x & 63) == 0 && vmax > 0.0) {
-            unsigned long long* dst = OP == OP_FNORM ? (unsigned long long*)&a.state[cur].fnorm : &a.state[cur].rnorm;
-            atomicMax(dst, (unsigned long long)__double_as_longlong(vmax));
-        }
+        if ((threadIdx.x & 63) == 0)
+            norm_max(OP == OP_FNORM ? (unsigned long long*)&a.state[cur].fnorm : &a.state[cur].rnorm, vmax);
         vmax = 0.0;
     };
     for (int it = i0; it < i1; it++) {

@@ -82,4 +82,16 @@ __device__ __forceinline__ T neighbour(const View<T>& u, const Faces<T>& F, int6
     return sign * F.two_h * g + u.at(a[0], a[1], a[2]);
 }
 
+// *norm = max(*norm, v) for v > 0 (bits of non-negative doubles order like the
+// doubles).  A norm's waves all hit one address, where atomics are served one
+// after the other: a wave whose value is no larger than what is there already
+// (a value read late is only smaller, never larger) leaves it at that.  About 12
+// ns per atomic: the FP64 norm-only residual of 257 x 257 x 129 57 -> 38 us, FP32
+// 48 -> 24 us, of 801 x 609 x 417 with 65536 waves 859 -> 654 us.
+__device__ __forceinline__ void norm_max(unsigned long long* norm, double v) {
+    if (!(v > 0.0)) return;
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+    if (bits > __hip_atomic_load(norm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(norm, bits);
+}
+
 }  // namespace mgp

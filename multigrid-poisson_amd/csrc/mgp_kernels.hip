@@ -90,7 +90,7 @@ __device__ __forceinline__ void block_max_into(double v, unsigned long long* out
     if (wave == 0) {
         double w = lane < nwaves ? part[lane] : 0.0;
         w = wave_max(w);
-        if (lane == 0 && w > 0.0) atomicMax(out, (unsigned long long)__double_as_longlong(w));
+        if (lane == 0) norm_max(out, w);
     }
 }
 

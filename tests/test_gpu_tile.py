@@ -99,6 +99,26 @@ def test_descents_equal_wave_march(shape, bc, sfx, points):
     np.testing.assert_array_equal(got[1], got[0])
 
 
+# a level of more points than "sweep.small_points": chunks of 6 planes at least
+def test_hilo_rows_give_the_same_bits():
+    shape, bc = (70, 66, 71), "NNNNDD"
+    dtype, halo, u0, f, faces, F, box = level(shape, bc, mgp.CONSISTENT, "f64", "hilo")
+    rng = np.random.default_rng(11)
+    new = lambda dt, v: mgp.DeviceArray(shape, halo, dtype=dt).upload(v)  # noqa: E731
+    hi, lo = new(np.float64, u0), new(np.float32, rng.standard_normal(u0.shape) * 1e-16)
+    e, r = new(np.float32, rng.standard_normal(u0.shape) * 1e-3), new(np.float64, rng.standard_normal(u0.shape))
+    got = []
+    for rows in (16, 8):
+        nrm = mgp.DeviceBuffer(np.zeros(1))
+        un, ln, out = (new(dt, np.ones(u0.shape)) for dt in (np.float64, np.float32, np.float32))
+        with tuned(update_residual__rows=rows):
+            mgp.call("mgp_update_residual_hilo_f64_f32", hi.ref(), un.ref(), lo.ref(), ln.ref(), e.ref(), f.ref(),
+                     r.ref(), out.ref(), ctypes.byref(F), mgp.box(box), nrm.ptr, None)
+        got.append([a.download() for a in (un, ln, out, nrm)])
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+
+
 # tiles of 16 rows x 124 columns; the three arrays with halos of their own
 @pytest.mark.parametrize("sfx", ["f64", "f32"])
 @pytest.mark.parametrize("mode", [mgp.REFERENCE, mgp.CONSISTENT])
@@ -137,3 +157,27 @@ def test_lds_sweeps_with_several_points_per_thread(mode, sfx, shape, bc):
         mgp.call("mgp_rbgs_sweep_" + sfx, mode, a.ref(), b.ref(), f.ref(), ctypes.byref(F), mgp.box(box), 0.93, None)
         a, b = b, a
     np.testing.assert_array_equal(c.download(), a.download())
+
+
+# boxes that leave planes, rows and columns outside, nothing, or everything
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("shape,box", [((9, 7, 70), (1, 8, 2, 6, 3, 69)), ((6, 5, 4), (0, 6, 0, 5, 0, 4)),
+                                       ((6, 5, 4), (2, 2, 1, 4, 1, 3)), ((20, 33, 65), (0, 19, 1, 33, 1, 64)),
+                                       ((7, 40, 3), (3, 7, 0, 40, 1, 2)), ((5, 6, 130), (1, 4, 5, 6, 0, 130))])
+def test_residual_norm_outside_the_box(shape, box, sfx):
+    dtype = np.float64 if sfx == "f64" else np.float32
+    rng = np.random.default_rng(zlib.crc32(repr((shape, box, sfx)).encode()))
+    u, f = (mgp.DeviceArray(shape, (1,) * 6, dtype=dtype) for _ in range(2))
+    for a in (u, f):
+        a.upload(rng.standard_normal(a.pshape))
+    r0 = rng.standard_normal(u.pshape)
+    for place in [(0, 0, 0), (shape[0] - 1, shape[1] - 1, shape[2] - 1), (shape[0] // 2, 0, 1), (1, shape[1] // 2, 0)]:
+        r0[1:-1, 1:-1, 1:-1][place] = 1e6 * (1 + sum(place))  # read where the box leaves it out
+        r = mgp.DeviceArray(shape, (1,) * 6, dtype=dtype)
+        for name in ("mgp_residual_", "mgp_residual_norm_"):
+            r.upload(r0)
+            nrm = mgp.DeviceBuffer(np.zeros(1))
+            mgp.call(name + sfx, mgp.CONSISTENT, u.ref(), f.ref(), r.ref(), mgp.box(box), 1.0, nrm.ptr, None)
+            if name == "mgp_residual_":
+                want = float(np.abs(r.download()[1:-1, 1:-1, 1:-1]).max())
+            assert nrm.download()[0] == want
