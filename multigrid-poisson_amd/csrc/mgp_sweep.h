@@ -49,6 +49,7 @@ template <class T>
 int march_jacobi(int mode, const mgp_array* u, const mgp_array* v, const mgp_array* f, const int64_t box[6],
                  double omega, double h, void* stream);
 extern int64_t g_jacobi_kernel;
+extern int64_t g_point_points;  // levels of fewer points: prolongation and stored residual per point
 // residual on a box through wave tiles (norm: max |r| over the whole shape
 // folded into *norm); MGP_ERR_ARG when the layouts do not allow it
 template <class T>

@@ -181,3 +181,25 @@ def test_residual_norm_outside_the_box(shape, box, sfx):
             if name == "mgp_residual_":
                 want = float(np.abs(r.download()[1:-1, 1:-1, 1:-1]).max())
             assert nrm.download()[0] == want
+
+
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("shape,bc", [((3, 3, 3), "NNNNNN"), ((5, 33, 17), "DDDDDD"), ((17, 9, 129), "NDDNDN"),
+                                      ((33, 35, 65), "NNNNDD")])
+def test_small_levels_per_point_equal_marches(shape, bc, sfx):
+    """Prolongation + add and the stored residual: the route of small levels
+    against the march."""
+    got = []
+    for points in (1 << 30, 0):
+        with tuned(small__point_points=points):
+            for mode in (mgp.REFERENCE, mgp.CONSISTENT):
+                dtype, halo, u0, f, faces, F, box = level(shape, bc, mgp.CONSISTENT, sfx, "small")
+                u, r = (mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0) for _ in range(2))
+                mgp.call("mgp_residual_" + sfx, mode, u.ref(), f.ref(), r.ref(), mgp.box(box), F.h, None, None)
+                got.append(r.download())
+            c = mgp.DeviceArray(tuple((v - 1) // 2 + 1 for v in shape), halo, dtype=dtype)
+            c.upload(np.random.default_rng(9).standard_normal(c.pshape))
+            mgp.call("mgp_prolong_add_" + sfx, c.ref(), u.ref(), None)
+            got.append(u.download())
+    for a, b in zip(got[:3], got[3:]):
+        np.testing.assert_array_equal(a, b)
