@@ -1,4 +1,6 @@
-// One-pass red-black Gauss-Seidel sweep for gfx950 (mgp_rbgs_sweep_*).
+// One-pass red-black Gauss-Seidel sweep for gfx950 (mgp_rbgs_sweep_*), and the
+// wave marches: sweeps where the workgroup tiles (mgp_tile.hip) and blocks
+// (mgp_block.hip) do not apply, residual, restriction and prolongation.
 //
 // The reference runs a sweep as two in-place half-sweeps over the whole
 // level, each preceded by a Neumann ghost refresh (include/relaxation.h:25-90,
