@@ -83,8 +83,9 @@ __device__ __forceinline__ void block_sweeps(const BlockArgs<T>& A, T (&sh)[2][B
     const int lin = MODE == MGP_MODE_REFERENCE ? (int)(A.lin0 & 1) : 0;
     const int s = (x + ys + z + lin) & 1;  // rows 2 q + s are red
     const int xc = min(x, n0 - 1), zc = min(z, n2 - 1);
-    // byte offsets within the arrays (of at most 2^24 points and their
-    // halos): row y of the block, clamped into the shape
+    // byte offsets within the arrays (from their first to their last point less
+    // than BUF_OOB, checked by the launch): row y of the block, clamped into the
+    // shape
     const uint32_t rowb = (uint32_t)(A.ui.s1 * (int64_t)sizeof(T));
     const uint32_t col = (uint32_t)(((int64_t)xc * A.ui.s0 + zc) * (int64_t)sizeof(T));
     const uint32_t row0 = col + (uint32_t)min(ys, n1 - 1) * rowb, rowl = col + (uint32_t)(n1 - 1) * rowb;
@@ -267,6 +268,13 @@ int block_sweep(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_ar
         if (f->stride[d] != ui->stride[d] || uo->stride[d] != ui->stride[d]) return MGP_ERR_ARG;
     const int64_t n[3] = {A.ui.n0, A.ui.n1, A.ui.n2};
     if (n[0] < 3 || n[1] < 2 || n[2] < 2 || n[0] * n[1] * n[2] > (int64_t)1 << 24) return MGP_ERR_ARG;
+    // u, f and the output are each addressed through one descriptor with 32-bit
+    // offsets, whose masked stores need BUF_OOB to lie past the array: a window
+    // into a larger array (strides wider than its shape) can span more.  The
+    // coarse level is addressed plane by plane
+    auto plane = [](const View<T>& v) { return ((v.n1 - 1) * v.s1 + v.n2) * (int64_t)sizeof(T); };
+    if ((n[0] - 1) * A.ui.s0 * (int64_t)sizeof(T) + plane(A.ui) >= (int64_t)BUF_OOB) return MGP_ERR_ARG;
+    if (coarse && plane(A.c) >= (int64_t)BUF_OOB) return MGP_ERR_ARG;
     for (int q = 0; q < 6; q++) {
         A.g[q] = faces->type[q] == MGP_NEUMANN ? static_cast<const T*>(faces->g[q]) : nullptr;
         if (faces->type[q] == MGP_NEUMANN && !A.g[q]) return MGP_ERR_ARG;

@@ -1,0 +1,58 @@
+"""Which kernel a call takes, checked on the CPU with the launches recorded
+instead of run: what a kernel's addresses cannot reach goes to one that can."""
+import pytest
+
+import launch_recorder
+
+NO_HALO = [0] * 6
+
+
+@pytest.fixture(scope="module")
+def recorder(tmp_path_factory):
+    return launch_recorder.build(str(tmp_path_factory.mktemp("recorder")))
+
+
+def sweep_call(kind, sfx, shape, strides=None, f_strides=None, c_strides=None, bc="DDDDDD", keys=None):
+    """mgp_rbgs_<kind>_<sfx> on arrays without halo (strides None: compact)."""
+    arrays = {"ui": (shape, NO_HALO, strides), "uo": (shape, NO_HALO, strides),
+              "f": (shape, NO_HALO, f_strides or strides),
+              "c": ([(n - 1) // 2 + 1 for n in shape], NO_HALO, c_strides)}
+    first = [1] + ([] if kind == "sweep2_from_zero" else ["ui"])
+    last = (["c"] if kind == "sweep2_prolong" else []) + ([3] if kind == "sweeps" else [])
+    box = [0 if bc[3] == "N" else 1, shape[0] - (bc[2] == "D"), 0 if bc[1] == "N" else 1, shape[1] - (bc[0] == "D"),
+           0 if bc[5] == "N" else 1, shape[2] - (bc[4] == "D")]
+    return {"name": "mgp_rbgs_%s_%s" % (kind, sfx), "arrays": arrays, "bc": bc, "box": box, "h": 1.0 / 16,
+            "args": first + ["uo", "f", "faces", "box", 0.93] + last + ["stream"], "keys": keys or {}}
+
+
+PAIRS = ["sweep2", "sweep2_prolong", "sweep2_from_zero"]
+
+
+# a window of `shape` in an array of n1 x n2 points per plane: its points are few
+# enough for blocks, its bytes from first to last are past what a 32-bit offset
+# with an out-of-range value left over can address
+@pytest.mark.parametrize("kind", PAIRS)
+@pytest.mark.parametrize("sfx,shape,n1,n2", [("f64", [129, 17, 33], 1025, 1025), ("f64", [129, 17, 33], 2049, 2049),
+                                             ("f32", [257, 17, 33], 1025, 1025), ("f64", [3, 9, 33], 4097, 16385)])
+def test_wide_windows_do_not_run_as_blocks(recorder, kind, sfx, shape, n1, n2):
+    size = 8 if sfx == "f64" else 4
+    wide = [n1 * n2, n2, 1]
+    span = ((shape[0] - 1) * wide[0] + (shape[1] - 1) * wide[1] + shape[2]) * size
+    assert span >= 1 << 30
+    # the same window with its planes just close enough, and compact
+    near = [((1 << 30) // size - (shape[1] - 1) * n2 - shape[2] - 1) // (shape[0] - 1), n2, 1]
+    calls = [sweep_call(kind, sfx, shape, s) for s in (wide, near, None)]
+    kernels = [[k[0] for k in ks] for rc, ks in launch_recorder.record(recorder, calls) if rc == 0]
+    assert ["k_rbgs_tile" in k[0] for k in kernels] == [True, False, False], kernels
+    assert ["k_rbgs_block" in k[0] for k in kernels] == [False, True, True], kernels
+
+
+def test_wide_coarse_planes_do_not_run_as_blocks(recorder):
+    """A coarse plane past 1 GiB is refused by the blocks as by the tiles and the
+    wave march: MGP_ERR_ARG, and nothing launched."""
+    shape = [17, 33, 33]
+    wide = [17 << 23, 1 << 23, 1]  # 16 rows on: 1 GiB in FP64
+    ok = [17 << 22, 1 << 22, 1]
+    r = launch_recorder.record(recorder, [sweep_call("sweep2_prolong", "f64", shape, c_strides=s) for s in (wide, ok)])
+    assert r[0] == (-1, [])
+    assert r[1][0] == 0 and "k_rbgs_block" in r[1][1][0][0]
