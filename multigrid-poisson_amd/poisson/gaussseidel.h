@@ -40,8 +40,19 @@ public:
         return d.settings.mode == CONSISTENT || ((d.u->stride[0] & 1) && (d.u->stride[1] & 1));
     }
 
+    // FP32 coarsest level of a refinement solve, its passes in FP64 arithmetic
+    // where the level fits one workgroup's LDS in doubles (u with a ghost layer and
+    // f in 64 KiB, so never more than 4096 points)
+    static bool coarsest_in_fp64(const Domain<T>& d) {
+        return std::is_same<T, float>::value && d.settings.coarse_fp64 && d.coarsest && !d.below;
+    }
+    static constexpr int64_t LDS_FP64_POINTS = 4096;
+
     void relax_level(Domain<T>& d, T omega, int_t nsmooth) override {
-        if (d.u_zero && from_zero(d, omega, nsmooth)) return;
+        // a hierarchy of one level starts its coarsest level from zero: no FP32
+        // pair in place of its FP64 passes
+        const bool lds = coarsest_in_fp64(d) && d.u->shape[0] * d.u->shape[1] * d.u->shape[2] <= LDS_FP64_POINTS;
+        if (d.u_zero && !lds && from_zero(d, omega, nsmooth)) return;
         d.materialize_zero();
         if (!d.u_alt || !d.settings.fused_sweeps || !checkerboard(d) || !alternate || nsmooth < 1) {
             Relaxation<T>::relax_level(d, omega, nsmooth);
@@ -57,11 +68,9 @@ public:
             const mgp_array ui = d.u->desc();
             mgp_array uo = ui;
             if (nsmooth & 1) uo.data = d.u_alt;
-            // FP32 coarsest level of a refinement solve: the passes in FP64
-            // arithmetic where the level fits the LDS in doubles
-            const bool dp = std::is_same<T, float>::value && d.settings.coarse_fp64 && d.coarsest && !d.below;
-            if (dp && mgp_rbgs_sweeps_f32_f64(d.settings.mode, &ui, &uo, &f, &F, b, (double)omega, nsmooth,
-                                              mgpx::stream()) == MGP_OK) {
+            if (coarsest_in_fp64(d) &&
+                mgp_rbgs_sweeps_f32_f64(d.settings.mode, &ui, &uo, &f, &F, b, (double)omega, nsmooth,
+                                        mgpx::stream()) == MGP_OK) {
                 if (nsmooth & 1) d.swap_u_alt();
                 return;
             }
