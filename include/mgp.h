@@ -188,8 +188,10 @@ int mgp_rbgs_half_f32(int mode, const mgp_array* u, const mgp_array* f, const in
  * leave in the shape; the halo of u_out is not written (ghosts are formed
  * again before every use).  Requires a
  * checkerboard colouring: always in consistent mode; in reference mode only
- * when stride[0] and stride[1] are odd (MGP_ERR_ARG otherwise).  An empty box
- * is a no-op in place and MGP_ERR_ARG out of place (nothing would be copied). */
+ * when stride[0] and stride[1] are odd (MGP_ERR_ARG otherwise).  f may have
+ * strides of its own.  MGP_ERR_ARG too for a plane of 4 GiB or more.  An empty
+ * box is a no-op in place and MGP_ERR_ARG out of place (nothing would be
+ * copied). */
 int mgp_rbgs_sweep_f64(int mode, const mgp_array* u_in, const mgp_array* u_out, const mgp_array* f,
                        const mgp_faces* faces, const int64_t box[6], double omega, void* stream);
 int mgp_rbgs_sweep_f32(int mode, const mgp_array* u_in, const mgp_array* u_out, const mgp_array* f,
@@ -199,9 +201,8 @@ int mgp_rbgs_sweep_f32(int mode, const mgp_array* u_in, const mgp_array* u_out, 
  * pairs of sweeps, include/gaussseidel.h:28-94 run twice per point; no
  * single counterpart in the reference), shape points outside the box copied
  * as above.  u_out must be a different buffer; MGP_ERR_ARG also where the
- * level has fewer than
- * 3 x-planes or a plane of 1 GiB or more (run single sweeps there), and for an
- * empty box. */
+ * level has fewer than 3 x-planes or a plane of 1 GiB or more or f has other
+ * strides than u_in (run single sweeps there), and for an empty box. */
 int mgp_rbgs_sweep2_f64(int mode, const mgp_array* u_in, const mgp_array* u_out, const mgp_array* f,
                         const mgp_faces* faces, const int64_t box[6], double omega, void* stream);
 int mgp_rbgs_sweep2_f32(int mode, const mgp_array* u_in, const mgp_array* u_out, const mgp_array* f,

@@ -73,6 +73,11 @@ extern int64_t g_sweep_min_chunk;
 static inline int64_t min_chunk_for(int64_t points) {
     return points < g_small_points ? g_small_min_chunk : g_sweep_min_chunk;
 }
+// b's points lie as a's do (the rows' stride counts only where there are two)
+template <class T>
+static inline bool same_strides(const View<T>& a, const View<T>& b) {
+    return a.s0 == b.s0 && (a.n1 == 1 || a.s1 == b.s1);
+}
 static inline int64_t box_points(const int64_t b[6]) { return (b[1] - b[0]) * (b[3] - b[2]) * (b[5] - b[4]); }
 
 namespace {
@@ -176,7 +181,9 @@ __global__ void __launch_bounds__(64 * (RH / NQ)) k_rbgs_march(MarchArgs<T> A) {
 
     // per owned position: element offset within a plane (clamped into the
     // shape so every load is valid), and masks
-    uint32_t off[NQ], foff[NQ];  // element offset in a plane; index in an x-face array
+    // byte offsets in a plane of u, in an x-face array, and in a plane of f
+    // (whose strides may differ from u's)
+    uint32_t off[NQ], foff[NQ], rhs[NQ];
     bool inb[NQ], core[NQ], inshape[NQ];
     int col0[NQ];
 #pragma unroll
@@ -187,8 +194,9 @@ __global__ void __launch_bounds__(64 * (RH / NQ)) k_rbgs_march(MarchArgs<T> A) {
         inb[q] = z_in && y >= A.by0 && y < A.by1;
         core[q] = inb[q] && z_core && rr >= 2 && rr <= TY + 1;
         const int64_t yc = min(max(y, (int64_t)0), n1 - 1), zc = min(max(z, (int64_t)0), n2 - 1);
-        off[q] = (uint32_t)((yc * s1 + zc) * (int64_t)sizeof(T));   // bytes
-        foff[q] = (uint32_t)((yc * n2 + zc) * (int64_t)sizeof(T));  // bytes
+        off[q] = (uint32_t)((yc * s1 + zc) * (int64_t)sizeof(T));
+        foff[q] = (uint32_t)((yc * n2 + zc) * (int64_t)sizeof(T));
+        rhs[q] = (uint32_t)((yc * A.f.s1 + zc) * (int64_t)sizeof(T));
         // colour at plane 0 (reference: parity of the halo-inclusive index,
         // include/gaussseidel.h:56,81; consistent: parity of i+j+k)
         col0[q] = MODE == MGP_MODE_REFERENCE ? (int)((A.lin0 + y * s1 + z) & 1) : (int)((y + z) & 1);
@@ -244,9 +252,9 @@ __global__ void __launch_bounds__(64 * (RH / NQ)) k_rbgs_march(MarchArgs<T> A) {
     };
     const T* fpl = A.f.p;
     auto load_f = [&](int64_t j, T (&dst)[NQ]) {
-        const T* pl = fpl + min(max(j, (int64_t)0), n0 - 1) * s0;
+        const T* pl = fpl + min(max(j, (int64_t)0), n0 - 1) * A.f.s0;
 #pragma unroll
-        for (int q = 0; q < NQ; q++) dst[q] = ld(pl, off[q]);
+        for (int q = 0; q < NQ; q++) dst[q] = ld(pl, rhs[q]);
     };
 
     T uo_m[NQ], uo_c[NQ], uo_p[NQ], uo_n[NQ], f_m[NQ], f_c[NQ], f_n[NQ], Pm2[NQ], Pm1[NQ], Pc[NQ];
@@ -1922,7 +1930,7 @@ int march_sweep(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_ar
     // wave tiles: planes addressed through buffer descriptors with a 32-bit
     // range (a plane must stay below the out-of-range lane offset)
     const int64_t plane_bytes = ((A.ui.n1 - 1) * A.ui.s1 + A.ui.n2) * (int64_t)sizeof(T);
-    if (g_sweep_kernel == 2 && A.ui.n0 >= 3 && plane_bytes < (int64_t)BUF_OOB) {
+    if (g_sweep_kernel == 2 && A.ui.n0 >= 3 && plane_bytes < (int64_t)BUF_OOB && same_strides(A.f, A.ui)) {
         // register rows per wave tile: measured best 12 (FP64) and 16 (FP32)
         // at 1025 x 1025 x 513
         const int rows = g_sweep_rows == 8 || g_sweep_rows == 12 || g_sweep_rows == 16 ? (int)g_sweep_rows
@@ -1947,6 +1955,9 @@ int march_sweep(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_ar
         const hipError_t e = hipGetLastError();
         return e == hipSuccess ? MGP_OK : (int)e;
     }
+    // k_rbgs_march: f by its own strides, 32-bit offsets within a plane
+    const int64_t fplane_bytes = ((A.f.n1 - 1) * A.f.s1 + A.f.n2) * (int64_t)sizeof(T);
+    if (std::max(plane_bytes, fplane_bytes) >= (int64_t)1 << 32) return MGP_ERR_ARG;
     const int threads = g_sweep_waves == 4 ? 256 : g_sweep_waves == 16 ? 1024 : 512;
     const dim3 g(A.ntiles_pad + complement_blocks(A.ui, b, threads));
     switch (g_sweep_waves) {
@@ -2359,7 +2370,8 @@ int march_sweep2(int mode, const mgp_array* ui, const mgp_array* uo, const mgp_a
     A.c = coarse ? view_of<T>(*coarse) : A.ui;
     // planes addressed through buffer descriptors with a 32-bit range
     const int64_t plane_bytes = ((A.ui.n1 - 1) * A.ui.s1 + A.ui.n2) * (int64_t)sizeof(T);
-    if (A.ui.n0 < 3 || plane_bytes >= (int64_t)BUF_OOB) return MGP_ERR_ARG;
+    // (f too, by u's strides)
+    if (A.ui.n0 < 3 || plane_bytes >= (int64_t)BUF_OOB || !same_strides(A.f, A.ui)) return MGP_ERR_ARG;
     if (coarse) {
         const int64_t cplane = ((A.c.n1 - 1) * A.c.s1 + A.c.n2) * (int64_t)sizeof(T);
         if (mode != MGP_MODE_CONSISTENT || cplane >= (int64_t)BUF_OOB || zero_in) return MGP_ERR_ARG;

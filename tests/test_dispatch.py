@@ -56,3 +56,39 @@ def test_wide_coarse_planes_do_not_run_as_blocks(recorder):
     r = launch_recorder.record(recorder, [sweep_call("sweep2_prolong", "f64", shape, c_strides=s) for s in (wide, ok)])
     assert r[0] == (-1, [])
     assert r[1][0] == 0 and "k_rbgs_block" in r[1][1][0][0]
+
+
+# f beside a u with a halo on every face: without one, with rows or planes
+# further apart
+F_LAYOUTS = {"no halo": lambda n: [n[1] * n[2], n[2], 1], "rows apart": lambda n: [(n[1] + 2) * (n[2] + 9), n[2] + 9, 1],
+             "planes apart": lambda n: [(n[1] + 40) * (n[2] + 2), n[2] + 2, 1]}
+
+
+@pytest.mark.parametrize("layout", list(F_LAYOUTS))
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("shape", [[5, 9, 33], [129, 33, 130]])
+def test_f_with_its_own_strides_is_not_read_by_u_strides(recorder, shape, sfx, layout):
+    """One sweep goes to the kernel that addresses f by its own strides; a pair,
+    which has none, is refused (single sweeps then)."""
+    calls = []
+    for kind in ["sweep"] + PAIRS:
+        c = sweep_call(kind, sfx, shape, bc="NNNNNN")
+        for name in ("ui", "uo", "c"):
+            c["arrays"][name] = (c["arrays"][name][0], [1] * 6, None)
+        c["arrays"]["f"] = (shape, NO_HALO, F_LAYOUTS[layout](shape))
+        calls.append(c)
+    got = launch_recorder.record(recorder, calls)
+    assert got[0][0] == 0 and len(got[0][1]) == 1 and "k_rbgs_march" in got[0][1][0][0], got[0]
+    assert got[1:] == [(-1, [])] * 3, got[1:]
+
+
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+def test_planes_past_32_bit_offsets_are_refused(recorder, sfx):
+    """A plane of u or f whose bytes do not fit 32-bit offsets: MGP_ERR_ARG."""
+    n2 = 1 << (25 if sfx == "f64" else 26)
+    wide, near, shape = [17 * n2, n2, 1], [17 * n2, n2 - 8, 1], [5, 17, 33]
+    calls = [sweep_call("sweep", sfx, shape, wide), sweep_call("sweep", sfx, shape, None, wide),
+             sweep_call("sweep", sfx, shape, near), sweep_call("sweep", sfx, shape, None, near)]
+    got = launch_recorder.record(recorder, calls)
+    assert got[:2] == [(-1, [])] * 2, got[:2]
+    assert all(rc == 0 and "k_rbgs_march" in k[0][0] for rc, k in got[2:]), got[2:]

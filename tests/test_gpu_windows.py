@@ -74,3 +74,32 @@ def test_sweeps_on_windows_equal_compact_levels(sfx, shape, bc, plane):
         np.testing.assert_array_equal(got[1], got[0])
         assert not np.array_equal(got[0][shape_slices(shape, halo)], other.astype(dtype)[shape_slices(shape, halo)])
     assert all(w.rest_is_untouched() for w in wide.values())
+
+
+# f without the halo u has (as a caller's right-hand side is stored), or with rows
+# or planes further apart: a sweep reads it by its own strides
+@pytest.mark.parametrize("f_halo,more", [((0,) * 6, None), ((1, 0, 0, 2, 0, 3), None), ((0,) * 6, (40, 9)),
+                                         (None, (11, 0))], ids=["none", "own", "window", "planes"])
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("mode", [mgp.REFERENCE, mgp.CONSISTENT])
+@pytest.mark.parametrize("shape,bc", [((3, 3, 3), "NNNNNN"), ((9, 31, 65), "NNNNNN"), ((17, 33, 127), "DNDNND"),
+                                      ((6, 29, 62), "DDNNDD"), ((65, 129, 65), "NNNNDD")])
+def test_sweep_reads_f_by_its_own_strides(shape, bc, mode, sfx, f_halo, more):
+    dtype = np.float64 if sfx == "f64" else np.float32
+    lv = random_level(shape, bc, mode, dtype, (shape, bc, mode, "f strides"))
+    if lv is None:
+        pytest.skip("reference colouring is not a checkerboard for this halo layout")
+    halo, u0, f, faces, F, box = lv
+    values = f.download()[shape_slices(shape, halo)]
+    f_halo = halo if f_halo is None else f_halo
+    own = np.full(mgp.padded_shape(shape, f_halo), 1e30)
+    own[shape_slices(shape, f_halo)] = values
+    dims = tuple(n + m for n, m in zip(own.shape, (0,) + (more or (0, 0))))
+    got = []
+    for rhs in (f, Window(own, shape, f_halo, dims, (0, dims[1] - own.shape[1], 0), dtype)):
+        a = mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0)
+        b = mgp.DeviceArray(shape, halo, dtype=dtype).upload(u0)
+        print("case f strides", shape, bc, mode, sfx, dims, flush=True)
+        mgp.call("mgp_rbgs_sweep_" + sfx, mode, a.ref(), b.ref(), rhs.ref(), ctypes.byref(F), mgp.box(box), 0.93, None)
+        got.append(b.download())
+    np.testing.assert_array_equal(got[1], got[0])
