@@ -628,7 +628,8 @@ int mgp_cycle_noalloc_f64(const char* cycle, const mgp_array* u, const mgp_array
  * FP64, bit 1 FP32; default 3), "residual.target_wgs",
  * "residual_fw.target_wgs", "prolong.target_wgs" (waves the norm-only
  * residual, the fused residual + full-weighting and the prolongation marches
- * aim for; 0 = the value of
+ * aim for, the fused march with running sums, which takes most levels, for
+ * twice as many; 0 = the value of
  * "sweep.target_wgs"; defaults 4096, 32768, 65536), "update_residual.target_wgs"
  * (waves of mgp_update_residual_f64_f32 and the hi + lo kernels, twice as many with
  * 8 rows; default 65536), "update_residual.rows" (8 or 16 register rows per wave

@@ -273,7 +273,7 @@ static int march_descend(const DescendArgs<T>& D, const mgp_array* u, const mgp_
     A.ztiles = (int32_t)((cf->shape[2] + MK - 1) / MK);
     const int64_t tiles = (int64_t)A.ytiles * A.ztiles;
     // (the march of mgp_sweep.hip aims for half as many)
-    int64_t chunks = std::max<int64_t>(1, 2 * g_fw_target / std::max<int64_t>(tiles, 1));
+    int64_t chunks = std::max<int64_t>(1, 2 * target_wgs(g_fw_target) / std::max<int64_t>(tiles, 1));
     chunks = std::min<int64_t>(chunks, std::max<int64_t>(1, c0 / 2));
     A.ichunk = (int32_t)((c0 + chunks - 1) / chunks);
     A.ntiles = (int32_t)(tiles * ((c0 + A.ichunk - 1) / A.ichunk));

@@ -55,8 +55,6 @@ int64_t g_prolong_target = 65536;
 // waves, 4.48 ms with 65536 (1025 x 1025 x 513); the hi + lo kernels aim for
 // twice as many with 8 rows
 int64_t g_upd_target = 65536;
-extern int64_t g_sweep_target_wgs;
-static inline int64_t target_wgs(int64_t own) { return own > 0 ? own : g_sweep_target_wgs; }
 
 // shortest x march of a launch over a box of `points` points: levels below
 // "sweep.small_points" points are latency-bound marches whose cost grows with

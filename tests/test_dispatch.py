@@ -92,3 +92,19 @@ def test_planes_past_32_bit_offsets_are_refused(recorder, sfx):
     got = launch_recorder.record(recorder, calls)
     assert got[:2] == [(-1, [])] * 2, got[:2]
     assert all(rc == 0 and "k_rbgs_march" in k[0][0] for rc, k in got[2:]), got[2:]
+
+
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+@pytest.mark.parametrize("shape", [[129, 129, 129], [257, 131, 70], [513, 513, 33]])
+def test_descent_march_takes_target_zero_as_the_sweeps_target(recorder, shape, sfx):
+    """"residual_fw.target_wgs" 0 means the value of "sweep.target_wgs": as many
+    waves as that value set directly, not one march per tile."""
+    coarse = [(n - 1) // 2 + 1 for n in shape]
+    arrays = {"u": (shape, [1] * 6, None), "f": (shape, [1] * 6, None), "r": (shape, [1] * 6, None),
+              "c": (coarse, NO_HALO, None)}
+    calls = [{"name": "mgp_residual_restrict_fw_" + sfx, "arrays": arrays, "bc": "NNNNNN", "h": 1.0 / 16,
+              "box": [0, shape[0], 0, shape[1], 0, shape[2]], "args": [1, "u", "f", "r", "c", "box", 1.0 / 16, "stream"],
+              "keys": {"residual_fw.target_wgs": target, "sweep.target_wgs": 20000}} for target in (0, 20000, 1)]
+    (zero, same, one) = (k for rc, k in launch_recorder.record(recorder, calls))
+    assert "k_resid_fw_march" in zero[0][0]
+    assert zero == same and zero[0][1] > 2 * one[0][1]
