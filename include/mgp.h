@@ -233,8 +233,8 @@ int mgp_rbgs_sweep2_from_zero_f64(int mode, const mgp_array* u_out, const mgp_ar
 int mgp_rbgs_sweep2_from_zero_f32(int mode, const mgp_array* u_out, const mgp_array* f, const mgp_faces* faces,
                                   const int64_t box[6], double omega, void* stream);
 /* nsweeps such sweeps in one launch, for a level small enough for one
- * workgroup's LDS ((nx+2)(ny+2)(nz+2) + nx ny nz elements <= 64 KiB;
- * MGP_ERR_ARG otherwise): the result of the last sweep goes to u_out, which may
+ * workgroup's LDS ((nx+2)(ny+2)(nz+2) + nx ny nz elements <= 64 KiB, no face
+ * of more than 1024 points; MGP_ERR_ARG otherwise): the result of the last sweep goes to u_out, which may
  * be u_in.  Same values as nsweeps calls of mgp_rbgs_sweep_* (the coarsest
  * level's smoothing, where launch latency dominates).  An empty box or
  * nsweeps = 0 is a no-op in place and MGP_ERR_ARG out of place. */

@@ -1043,11 +1043,15 @@ static int rbgs_sweep2_from_zero(int mode, const mgp_array* uo, const mgp_array*
     return march_sweep2<T>(mode, uo, uo, f, faces, b, omega, stream, nullptr, true);
 }
 
-// LDS bytes the multi-sweep kernel needs for a level, 0 when it does not fit
-static inline size_t lds_sweeps_bytes(const mgp_array* u, size_t esize) {
-    const size_t b = ((size_t)(u->shape[0] + 2) * (u->shape[1] + 2) * (u->shape[2] + 2) +
-                      (size_t)u->shape[0] * u->shape[1] * u->shape[2]) * esize;
-    return b <= 65536 ? b : 0;
+// levels the multi-sweep kernel takes: u with a ghost layer and f within 64 KiB
+// (as if f were in LDS too), no face of more than 1024 points.  It needs less
+// than a level of that size may take: at most 82000 bytes of the 160 KiB a
+// workgroup can have (FP64 408 x 2 x 2, its rows and planes padded to odd
+// lengths), at most 2048 (FP64) or 4096 (FP32) points of a colour
+static inline bool lds_sweeps_fit(const mgp_array* u, size_t esize) {
+    const int64_t n0 = u->shape[0], n1 = u->shape[1], n2 = u->shape[2];
+    return ((size_t)(n0 + 2) * (n1 + 2) * (n2 + 2) + (size_t)n0 * n1 * n2) * esize <= 65536 && n1 * n2 <= 1024 &&
+           n0 * n2 <= 1024 && n0 * n1 <= 1024;
 }
 
 template <class S, class T = S>
@@ -1071,19 +1075,15 @@ static int rbgs_sweeps(int mode, const mgp_array* ui, const mgp_array* uo, const
         return MGP_ERR_ARG;
     for (int q = 0; q < 6; q++)
         if (faces->type[q] == MGP_NEUMANN && !faces->g[q]) return MGP_ERR_ARG;
-    const size_t lds = lds_sweeps_bytes(ui, sizeof(T));
-    if (!lds) return MGP_ERR_ARG;  // too large for one workgroup
-    if ((b[1] - b[0]) * (b[3] - b[2]) * (b[5] - b[4]) > 8 * 1024) return MGP_ERR_ARG;  // 8 points per thread
+    if (!lds_sweeps_fit(ui, sizeof(T))) return MGP_ERR_ARG;  // too large for one workgroup
     const int64_t n0 = ui->shape[0], n1 = ui->shape[1], n2 = ui->shape[2];
-    if (n1 * n2 > 1024 || n0 * n2 > 1024 || n0 * n1 > 1024) return MGP_ERR_ARG;  // one ghost per thread and face
     if (box_empty(bx) || nsweeps == 0) return ui->data == uo->data ? MGP_OK : MGP_ERR_ARG;
     const RelaxConsts<T> c(omega, faces->h);
     const Faces<S> F = faces_of<S>(*faces);
     const T two_h = (T)(2.0 * faces->h);  // include/neumann.h:108, in the arithmetic type
     const View<S> vi = view_of<S>(*ui);
     const hipStream_t s = (hipStream_t)stream;
-    // red (and black) points, the box's rows and planes padded to odd lengths:
-    // at most 2048 in FP64 and 4096 in FP32, by the limit on the level above
+    // red (and black) points, the box's rows and planes padded to odd lengths
     const int64_t pts = ((b[1] - b[0]) * ((b[3] - b[2]) | 1) * ((b[5] - b[4]) | 1) + 1) / 2;
     const dim3 blk((unsigned)std::min<int64_t>(1024, (pts + 63) / 64 * 64));
     const size_t bytes = ((size_t)(n0 + 2) * ((n1 + 2) | 1) * ((n2 + 2) | 1) + 1) / 2 * 2 * sizeof(T);
@@ -1097,11 +1097,9 @@ static int rbgs_sweeps(int mode, const mgp_array* ui, const mgp_array* uo, const
     } else if (pts <= 2048) {
         if (ref) MGP_LDS_LAUNCH(MGP_MODE_REFERENCE, 2);
         else MGP_LDS_LAUNCH(MGP_MODE_CONSISTENT, 2);
-    } else if (pts <= 4096) {
+    } else {  // FP32
         if (ref) MGP_LDS_LAUNCH(MGP_MODE_REFERENCE, 4);
         else MGP_LDS_LAUNCH(MGP_MODE_CONSISTENT, 4);
-    } else {
-        return MGP_ERR_ARG;
     }
 #undef MGP_LDS_LAUNCH
     return launch_status();
