@@ -640,7 +640,8 @@ int mgp_cycle_noalloc_f64(const char* cycle, const mgp_array* u, const mgp_array
  * and full-weighting restriction; 0 = 6, default), "residual_fw.depth" (1 or
  * 2 fine planes of loads in flight per wave; 0 = 1 for FP64 and 2 for FP32,
  * default),
- * "jacobi.kernel" (1: per-point kernel; 2: wave tiles marching along x, default),
+ * "jacobi.kernel" (1: per-point kernel; 2: wave tiles marching along x; 0: by the
+ * size of the box, default),
  * "small.point_points" (levels of fewer points take the per-point kernels for
  * mgp_prolong_add_* and for mgp_residual_* without a norm; default 3 * 2^19),
  * "prolong.kernel" (1: per-point kernel; 2: wave tiles marching along x for

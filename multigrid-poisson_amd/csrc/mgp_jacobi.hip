@@ -13,8 +13,9 @@
 // Measured against one thread per point (1: k_jacobi), with the ghost refresh:
 // 385 x 353 x 321 FP64 0.234 / 0.315 ms (1.05 GB moved, 4.6 TB/s), FP32 0.129 /
 // 0.184; 1025 x 1025 x 513 3.35 / 3.52 and 1.64 / 2.11; 801 x 609 x 417 1.24 /
-// 1.52 and 0.62 / 0.90; 257 x 257 x 129 41 / 72 and 30 / 41 us; the same within
-// 1 us at 129 x 129 x 65 and 65 x 65 x 33.
+// 1.52 and 0.62 / 0.90; 257 x 257 x 129 41 / 72 and 30 / 41 us.  Small boxes and
+// those that fill little of the tiles' 16 rows x 124 columns are left to one
+// thread per point (march_pays).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,7 +29,7 @@
 
 namespace mgp {
 
-int64_t g_jacobi_kernel = 2;  // 1: one thread per point, 2: wave tiles marching along x
+int64_t g_jacobi_kernel = 0;  // 1: one thread per point, 2: wave tiles marching along x, 0: by the box
 
 namespace {
 
@@ -125,6 +126,27 @@ __global__ void __launch_bounds__(64 * NW) k_jacobi_march(JacobiArgs<T> A) {
     else jacobi_march<T, MODE, R, NW, false>(A, tl);
 }
 
+// Where the march is the faster one.  Below 2^20 (FP64) or 2^21 (FP32) box points
+// either kernel is a few us, most of it the launch and one trip to memory, and
+// the march adds its chain of planes: per point / march, us, without the ghost
+// refresh, 33 x 33 x 33 FP64 4.2 / 4.9, 65 x 65 x 33 FP32 4.2 / 5.0, 128 x 128 x
+// 65 FP32 4.9 / 7.0.  Lanes and rows of a tile outside the box cost as much as
+// those inside.  FP32: the box has to fill half of its tiles (707 x 707 x 33
+// 69.7 / 80.6, 2^22 points by 17 columns 33 / 46; 2^21 points by 129 columns 10.3 /
+// 9.0, 2^22 by 65 17.0 / 14.9).  FP64, twice the bytes for the same lanes: a third
+// of them below 2^21 points (1025 x 33 x 33 9.9 / 13.3, 128 x 128 x 65 8.0 / 7.4),
+// any box above (2^21 points by 9 columns 51.0 / 48.9, 707 x 707 x 33 176 / 144).
+// Of 1541 random boxes of up to 1100 points a side the rule sends 533 to the
+// march, which gains 33 % (FP64) and 54 % (FP32) on average there; 7 of them, FP64,
+// take 3 to 15 % longer.  The others would on average have taken 14 and 17 % longer.
+template <class T>
+static bool march_pays(int64_t nx, int64_t ny, int64_t nz) {
+    const int64_t points = nx * ny * nz, area = ny * nz;
+    const int64_t tiles = (ny + 15) / 16 * 16 * ((nz + 123) / 124 * 124);
+    if (sizeof(T) == 8) return points >= (int64_t)1 << (3 * area >= tiles ? 20 : 21);
+    return points >= (int64_t)1 << 21 && 2 * area >= tiles;
+}
+
 }  // namespace
 
 template <class T>
@@ -133,6 +155,7 @@ int march_jacobi(int mode, const mgp_array* u, const mgp_array* v, const mgp_arr
     constexpr int R = 4, NW = 4;
     const int64_t nx = b[1] - b[0], ny = b[3] - b[2], nz = b[5] - b[4];
     if (nx < 1 || ny < 1 || nz < 2) return MGP_ERR_ARG;
+    if (g_jacobi_kernel == 0 && !march_pays<T>(nx, ny, nz)) return MGP_ERR_ARG;
     if (u->data == v->data) return MGP_ERR_ARG;  // (a march reads planes ahead of what it writes)
     JacobiArgs<T> A;
     const mgp_array* a[3] = {u, v, f};

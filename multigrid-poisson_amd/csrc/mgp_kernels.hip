@@ -1151,7 +1151,7 @@ static int jacobi(int mode, const mgp_array* u, const mgp_array* v, const mgp_ar
     const Box bx = box_of(b);
     if (box_empty(bx)) return MGP_OK;
     if (mode != MGP_MODE_REFERENCE && mode != MGP_MODE_CONSISTENT) return MGP_ERR_ARG;
-    if (g_jacobi_kernel == 2 && march_jacobi<T>(mode, u, v, f, b, omega, h, stream) == MGP_OK) return MGP_OK;
+    if (g_jacobi_kernel != 1 && march_jacobi<T>(mode, u, v, f, b, omega, h, stream) == MGP_OK) return MGP_OK;
     const BoxGrid g = box_grid(bx);
     const RelaxConsts<T> c(omega, h);
     if (mode == MGP_MODE_REFERENCE)

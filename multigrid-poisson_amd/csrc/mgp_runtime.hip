@@ -137,7 +137,7 @@ int mgp_tuning_set(const char* key, int64_t value) {
     else if (!strcmp(key, "sweep.tile") && value <= 3) mgp::g_tile = value;
     else if (!strcmp(key, "sweep2.blocks") && value <= (1 << 20)) mgp::g_block_count = value;
     else if (!strcmp(key, "small.point_points")) mgp::g_point_points = value;
-    else if (!strcmp(key, "jacobi.kernel") && (value == 1 || value == 2)) mgp::g_jacobi_kernel = value;
+    else if (!strcmp(key, "jacobi.kernel") && value <= 2) mgp::g_jacobi_kernel = value;
     else if (!strcmp(key, "residual_fw.block_points") && value <= (1 << 24)) mgp::g_fw_block_points = value;
     else if (!strcmp(key, "sweep.pair") && (value == 0 || value == 1)) mgp::g_sweep_pair = value;
     else if (!strcmp(key, "sweep2.rows") &&

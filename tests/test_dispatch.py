@@ -108,3 +108,26 @@ def test_descent_march_takes_target_zero_as_the_sweeps_target(recorder, shape, s
     (zero, same, one) = (k for rc, k in launch_recorder.record(recorder, calls))
     assert "k_resid_fw_march" in zero[0][0]
     assert zero == same and zero[0][1] > 2 * one[0][1]
+
+
+def jacobi_call(sfx, shape, keys=None):
+    arrays = {n: (shape, [1] * 6, None) for n in "uvf"}
+    return {"name": "mgp_jacobi_" + sfx, "arrays": arrays, "bc": "NNNNNN", "h": 1.0, "keys": keys or {},
+            "box": [0, shape[0], 0, shape[1], 0, shape[2]],
+            "args": [1, "u", "v", "f", "box", 0.9, 1.0, "stream"]}
+
+
+# box sizes on both sides of the rule: points, and (FP32) how much of 16 rows x
+# 124 columns per tile the box fills
+@pytest.mark.parametrize("sfx,shape,march", [
+    ("f64", [33, 33, 33], False), ("f64", [56, 332, 34], False), ("f64", [127, 128, 64], False),
+    ("f64", [128, 128, 64], True), ("f64", [1025, 33, 33], False), ("f64", [2049, 33, 33], True),
+    ("f64", [1025, 32, 41], False), ("f64", [1025, 32, 42], True), ("f64", [385, 353, 321], True),
+    ("f32", [65, 65, 65], False), ("f32", [127, 128, 128], False), ("f32", [128, 128, 128], True),
+    ("f32", [359, 125, 61], False), ("f32", [1024, 512, 61], False), ("f32", [1024, 512, 62], True),
+    ("f32", [1024, 17, 248], True), ("f32", [1024, 17, 220], False), ("f32", [707, 707, 33], False)])
+def test_jacobi_march_where_it_pays(recorder, sfx, shape, march):
+    calls = [jacobi_call(sfx, shape), jacobi_call(sfx, shape, {"jacobi.kernel": 2}),
+             jacobi_call(sfx, shape, {"jacobi.kernel": 1})]
+    names = [k[0][0] for rc, k in launch_recorder.record(recorder, calls)]
+    assert ["k_jacobi_march" in n for n in names] == [march, True, False], names
