@@ -642,8 +642,9 @@ int mgp_cycle_noalloc_f64(const char* cycle, const mgp_array* u, const mgp_array
  * default),
  * "jacobi.kernel" (1: per-point kernel; 2: wave tiles marching along x; 0: by the
  * size of the box, default),
- * "small.point_points" (levels of fewer points take the per-point kernels for
- * mgp_prolong_add_* and for mgp_residual_* without a norm; default 3 * 2^19),
+ * "small.point_points" (levels of fewer points, and of fewer than 5/3 as many
+ * lanes at 64 to a row, take the per-point kernels for mgp_prolong_add_* and for
+ * mgp_residual_* without a norm; default 3 * 2^19),
  * "prolong.kernel" (1: per-point kernel; 2: wave tiles marching along x for
  * mgp_prolong_add_*, default), "batch.blocks" (workgroups per launch of the
  * batched solver's work lists, default 16384).

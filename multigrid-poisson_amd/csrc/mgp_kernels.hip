@@ -1173,6 +1173,13 @@ static int jacobi(int mode, const mgp_array* u, const mgp_array* v, const mgp_ar
 // (With a norm the march is the faster one at every size: 9.0 against 38 us at 65 x
 // 65 x 65.)
 int64_t g_point_points = (int64_t)3 << 19;
+// (a launch per point has 64 lanes per row of z, however few columns there are: a
+// level so narrow or ragged that they make five thirds of that many lanes marches.
+// 359 x 279 x 11 FP32, prolongation 22.0 / 13.1, 125 x 733 x 15 FP64 23.0 / 14.9;
+// residual 646 x 258 x 9 FP64 37.5 / 28.8, 469 x 46 x 70 13.5 / 12.5)
+static inline bool per_point(int64_t points, const BoxGrid& g) {
+    return points < g_point_points && (int64_t)g.grid.x * g.grid.y * (BZ * BY) / 5 * 3 < g_point_points;
+}
 
 template <class T>
 static int residual(int mode, const mgp_array* u, const mgp_array* f, const mgp_array* r, const int64_t b[6], double h,
@@ -1181,7 +1188,7 @@ static int residual(int mode, const mgp_array* u, const mgp_array* f, const mgp_
         !valid_box(u, b) || (mode != MGP_MODE_REFERENCE && mode != MGP_MODE_CONSISTENT))
         return MGP_ERR_ARG;
     const Box bx = box_of(b);
-    const bool small = !norm && u->shape[0] * u->shape[1] * u->shape[2] < g_point_points;
+    const bool small = !norm && !box_empty(bx) && per_point(u->shape[0] * u->shape[1] * u->shape[2], box_grid(bx));
     if (g_resid_kernel == 2 && !small && march_residual<T>(mode, u, f, r, b, h, norm, stream) == MGP_OK) return MGP_OK;
     const T hsq = (T)(h * h);  // include/residual.h:23
     const T inv_h2 = (T)(1.0 / (h * h));
@@ -1233,12 +1240,11 @@ static int prolong(const mgp_array* coarse, const mgp_array* fine, void* stream)
     if (!valid_array(coarse) || !valid_array(fine)) return MGP_ERR_ARG;
     for (int d = 0; d < 3; d++)  // exact 2:1 nesting (trilinearinterpolation.h:31-37)
         if (2 * (coarse->shape[d] - 1) + 1 != fine->shape[d]) return MGP_ERR_ARG;
-    const int64_t points = fine->shape[0] * fine->shape[1] * fine->shape[2];
-    if (ADD && g_prolong_kernel == 2 && points >= g_point_points &&
-        march_prolong_add<T>(coarse, fine, stream) == MGP_OK)
-        return MGP_OK;
     const Box bx = shape_box(fine);
     const BoxGrid g = box_grid(bx);
+    if (ADD && g_prolong_kernel == 2 && !per_point(fine->shape[0] * fine->shape[1] * fine->shape[2], g) &&
+        march_prolong_add<T>(coarse, fine, stream) == MGP_OK)
+        return MGP_OK;
     hipLaunchKernelGGL((k_prolong<T, ADD>), g.grid, g.block, 0, (hipStream_t)stream, view_of<T>(*coarse),
                        view_of<T>(*fine), bx, g.zchunks);
     return launch_status();

@@ -131,3 +131,24 @@ def test_jacobi_march_where_it_pays(recorder, sfx, shape, march):
              jacobi_call(sfx, shape, {"jacobi.kernel": 1})]
     names = [k[0][0] for rc, k in launch_recorder.record(recorder, calls)]
     assert ["k_jacobi_march" in n for n in names] == [march, True, False], names
+
+
+# levels on both sides of the rule: 3 * 2^19 points, and 5 * 2^19 lanes with the
+# rows of z filled up to 64
+@pytest.mark.parametrize("shape,per_point", [
+    ([65, 65, 65], True), ([129, 129, 65], True), ([33, 33, 17], True), ([45, 73, 309], True), ([129, 129, 129], False),
+    ([105, 381, 13], True), ([109, 381, 13], False), ([359, 279, 11], False), ([125, 733, 15], False), ([647, 257, 9], False)])
+@pytest.mark.parametrize("sfx", ["f64", "f32"])
+def test_small_levels_per_point_unless_narrow(recorder, sfx, shape, per_point):
+    coarse = [(n - 1) // 2 + 1 for n in shape]
+    box = [0, shape[0], 0, shape[1], 0, shape[2]]
+    calls = []
+    for keys in ({}, {"small.point_points": 0}, {"small.point_points": 1 << 30}):
+        base = {"bc": "NNNNNN", "h": 1.0, "box": box, "keys": keys}
+        calls.append({"name": "mgp_prolong_add_" + sfx, "args": ["c", "u", "stream"],
+                      "arrays": {"c": (coarse, NO_HALO, None), "u": (shape, NO_HALO, None)}, **base})
+        calls.append({"name": "mgp_residual_" + sfx, "args": [1, "u", "f", "r", "box", 1.0, None, "stream"],
+                      "arrays": {n: (shape, [1] * 6, None) for n in "ufr"}, **base})
+    names = [k[0][0] for rc, k in launch_recorder.record(recorder, calls)]
+    marches = ["_wave" in n for n in names]
+    assert marches == [not per_point] * 2 + [True] * 2 + [False] * 2, names
