@@ -610,9 +610,10 @@ int mgp_cycle_noalloc_f64(const char* cycle, const mgp_array* u, const mgp_array
  * or "sweep2.rows" and "sweep2.pack", have their defaults; default 3),
  * "sweep2.blocks" (two sweeps of a level that this many blocks of 16 planes x 12
  * (FP64) or 16 (FP32) rows x 64 columns cover run as blocks, one workgroup each,
- * under the same keys; default 256, 0: none), "residual_fw.block_points" (fine levels of at most this many
- * points take the fused residual and full-weighting restriction in blocks
- * while "residual_fw.rows" and "residual_fw.depth" are 0; default 2^21),
+ * under the same keys; default 256, 0: none), "residual_fw.block_points" (fine
+ * levels of at most this many points, but for narrow ones in FP64, take the fused
+ * residual and full-weighting restriction in blocks while "residual_fw.rows" and
+ * "residual_fw.depth" are 0; default 2^21),
  * "sweep.small_points" and
  * "sweep.small_min_chunk" (levels with fewer points than the first use the
  * second as their shortest x march; defaults 2^18 and 1), "sweep2.rows"

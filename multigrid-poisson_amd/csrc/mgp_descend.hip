@@ -105,9 +105,8 @@ __global__ void __launch_bounds__(64 * DW) k_resid_fw_block(DescendArgs<T> A) {
 // 257 x 129 FP64 54 / 65, FP32 33 / 41; 513 x 513 x 257 348 / 356, 184 / 200;
 // 1025 x 1025 x 513 FP32 1363 / 1423.  There both are bound by the memory
 // traffic of the shared rows: short marches (many waves close together in x)
-// beat fewer warm-up planes, and the FP64 level keeps the taller tiles of the
-// other march (2.63 / 2.60 ms); waves of a workgroup kept in step by a barrier
-// per plane were slower (2.73-3.39 ms).
+// beat fewer warm-up planes; waves of a workgroup kept in step by a barrier
+// per plane were slower (2.73-3.39 ms at 1025 x 1025 x 513 FP64).
 template <class T>
 struct MarchDescendArgs : DescendArgs<T> {
     int32_t ylo, yhi, zlo, zhi, xlo, xhi;  // allocated index ranges of the fine arrays
@@ -299,11 +298,21 @@ int block_residual_fw(const mgp_array* u, const mgp_array* f, const mgp_array* r
     A.bz0 = (int32_t)b[4], A.bz1 = (int32_t)b[5];
     A.inv_h2 = (T)(1.0 / (h * h));
     const int64_t pts = u->shape[0] * u->shape[1] * u->shape[2];
-    if (sizeof(T) == 8 && pts >= (int64_t)1 << 27) return MGP_ERR_ARG;  // the taller tiles: 2.60 / 2.63 ms
-    if (pts > g_fw_block_points) return march_descend<T>(A, u, cf, stream);
+    // Large FP64 levels keep the taller tiles of mgp_sweep.hip, which re-read fewer
+    // rows.  Running sums / taller tiles, us, over 70 random sizes from 2.5e7 points
+    // on: below 5 * 2^24 points 1.5 % more to 11 % less (683 x 265 x 181 221 / 245, 513 x
+    // 513 x 257 348 / 355), above from 2 % less to 11 % more (195 x 613 x 893 683 /
+    // 616, 483 x 525 x 407 537 / 505, 1025 x 1025 x 513 2631 / 2598)
+    if (sizeof(T) == 8 && pts >= (int64_t)5 << 24) return MGP_ERR_ARG;
     const int64_t xt = (cf->shape[0] + DC - 1) / DC;
     A.ytiles = (int32_t)((cf->shape[1] + DC - 1) / DC);
     A.ztiles = (int32_t)((cf->shape[2] + DK - 1) / DK);
+    // FP64 blocks of which at most half the lanes have a coarse column, on levels that
+    // take more than two of them per CU: march / blocks, us, 233 x 303 x 11 19.2 /
+    // 27.3, 895 x 89 x 25 23.2 / 33.3, 443 x 89 x 17 14.8 / 18.1, 301 x 301 x 17 24.6 /
+    // 33.4 (filled ones, 129 x 129 x 125: 20.4 / 19.0)
+    const bool narrow = sizeof(T) == 8 && cf->shape[2] <= DK / 2 && xt * A.ytiles > 512;
+    if (pts > g_fw_block_points || narrow) return march_descend<T>(A, u, cf, stream);
     hipLaunchKernelGGL(k_resid_fw_block<T>, dim3((unsigned)(xt * A.ytiles * A.ztiles)), dim3(64 * DW), 0,
                        (hipStream_t)stream, A);
     const hipError_t e = hipGetLastError();

@@ -152,3 +152,20 @@ def test_small_levels_per_point_unless_narrow(recorder, sfx, shape, per_point):
     names = [k[0][0] for rc, k in launch_recorder.record(recorder, calls)]
     marches = ["_wave" in n for n in names]
     assert marches == [not per_point] * 2 + [True] * 2 + [False] * 2, names
+
+
+# levels on both sides of each line: 2^21 points, 512 blocks with at most half
+# their columns, 5 * 2^24 points (the last two in FP64)
+@pytest.mark.parametrize("shape,f64,f32", [
+    ([65, 65, 33], "block", "block"), ([129, 129, 125], "block", "block"), ([129, 129, 129], "march", "march"),
+    ([233, 303, 11], "march", "block"), ([121, 257, 31], "march", "block"), ([121, 257, 33], "block", "block"),
+    ([121, 251, 31], "block", "block"), ([513, 513, 257], "march", "march"), ([483, 525, 407], "wave", "march"),
+    ([511, 513, 319], "march", "march"), ([513, 513, 319], "wave", "march"), ([1025, 1025, 513], "wave", "march")])
+def test_descent_kernel_by_size(recorder, shape, f64, f32):
+    coarse = [(n - 1) // 2 + 1 for n in shape]
+    calls = [{"name": "mgp_residual_restrict_fw_" + sfx, "bc": "NNNNNN", "h": 1.0,
+              "arrays": {**{n: (shape, [1] * 6, None) for n in "ufr"}, "c": (coarse, NO_HALO, None)},
+              "box": [0, shape[0], 0, shape[1], 0, shape[2]], "args": [1, "u", "f", "r", "c", "box", 1.0, "stream"]}
+             for sfx in ("f64", "f32")]
+    names = [k[0][0] for rc, k in launch_recorder.record(recorder, calls)]
+    assert all("k_resid_fw_" + want in name for name, want in zip(names, (f64, f32))), names
