@@ -22,10 +22,11 @@
 //
 // Measured against the tiles' march, us (two sweeps / with the correction):
 // 65 x 65 x 33 with Neumann x and y faces FP64 24 -> 15 / 32 -> 20, FP32 21 -> 12
-// / 25 -> 14; 33^3 FP64 23 -> 11 / 32 -> 17.  The work of the rings is 4 times
-// that of the points, so a launch takes this form while one block per CU covers
-// the level: 129 x 129 x 65 (992 blocks in FP64) takes 61 / 91 us, the march 39 /
-// 47.
+// / 25 -> 14; 33^3 FP64 23 -> 11 / 32 -> 17.  A block inside the level holds 12288
+// (FP64) or 16384 (FP32) points to write 8 x 4 x 56 = 1792 or 8 x 8 x 56 = 3584, its
+// rings 5.9 or 3.6 times that, so a launch takes this form while one block per CU
+// covers the level: 129 x 129 x 65 (992 blocks in FP64) takes 61 / 91 us, the march
+// 39 / 47.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -63,9 +63,13 @@ int64_t g_upd_target = 65536;
 int64_t g_small_points = 1 << 18;
 int64_t g_small_min_chunk = 1;
 // the Gauss-Seidel smoother pairs its sweeps (mgp_rbgs_sweep2_*) on levels of
-// at least this many points: every level.  FP64, Neumann x and y faces, pair /
-// two sweeps: 257 x 257 x 129 84 / 104 us, 129 x 129 x 65 39 / 35 us (with the
-// correction inside 47 / 47 us and one launch less), 65 x 65 x 33 15 / 22 us
+// at least this many points: every level.  Pair / two sweeps, us, Neumann x and y
+// faces: FP64 257 x 257 x 129 84 / 102, 65 x 65 x 33 15 / 21, FP32 56 / 71, 12 / 19.
+// Around a million points, where tiles have chunks of a few planes, it is close,
+// and two sweeps win at some sizes: FP64 129 x 129 x 65 38.6 / 33.0, with Dirichlet
+// faces 33.8 / 32.9, 161 x 161 x 81 41.9 / 41.3 and 41.3 / 37.1, FP32 129 x 129 x 65
+// 31.1 / 28.0 and 26.3 / 28.2.  (The pair after a coarse level takes the correction in
+// its stride, 47 us against 33 and a launch of 11 at 129 x 129 x 65 FP64.)
 int64_t g_pair_min_points = 0;
 extern int64_t g_sweep_min_chunk;
 static inline int64_t min_chunk_for(int64_t points) {
@@ -2121,9 +2125,12 @@ int march_update_residual(int mode, const mgp_array* u, const mgp_array* un, con
 // rows per wave tile of the hi + lo update + residual: 8 or 16.  At 8 the march
 // runs two waves per SIMD instead of one, and twice as many waves share the
 // planes in flight; x chunks of 6 planes at least.  FP64 update + residual,
-// 8 rows / 16 rows: 1025 x 1025 x 513 5.60 / 6.05 ms (21.6 GB moved: 3.9 TB/s),
-// 801 x 609 x 417 2.40 / 2.65 ms, 513 x 513 x 257 757 / 762 us (774 with chunks
-// of 4 planes), 257 x 257 x 129 125 / 129 us.  Measured and left: two columns
+// 8 rows / 16 rows in turn on the same buffers: 1025 x 1025 x 513 5.63 / 6.02 ms
+// (21.6 GB moved: 3.8 TB/s), 801 x 609 x 417 2.40 / 2.66 ms, 449 x 449 x 225 518 / 525
+// us, 257 x 257 x 129 110 / 113, 129 x 129 x 129 28 / 36; 513 x 513 x 257 787 / 762 with
+// Dirichlet faces, 744 / 755 with Neumann x and y faces.  Where the eight arrays lie
+// in memory counts for more than the rows on large levels: 4.6 to 5.6 ms / 4.8 to
+// 6.0 ms over other buffers at 1025 x 1025 x 513.  Measured and left: two columns
 // per lane on 4 rows, four waves to a workgroup (6.29 ms, 2.37 ms, 803 us, 155
 // us: the ghosts of both columns spill), the same on 8 rows (5.93 ms, 2.32 ms,
 // 855 us, 172 us).
