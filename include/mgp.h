@@ -414,7 +414,9 @@ int mgp_solver_stats(void* solver, double* rel_res, double* seconds, int64_t* it
 /* host mirror and device descriptor of level `level`'s u ('u'), uprev ('p'),
  * f ('f') or r ('r'); for MGP_MIXED also 'l': the FP32 lo word of the hi + lo
  * iterate on level 0 (device only, *host = NULL; MGP_ERR_ARG with
- * MGP_SOLVER_PLAIN_ITERATE) */
+ * MGP_SOLVER_PLAIN_ITERATE).  Smoothing out of place leaves u (and 'l') in
+ * either of two buffers: take the descriptor again after a call that solves or
+ * runs cycles */
 int mgp_solver_array(void* solver, int level, int which, void** host, mgp_array* device);
 /* host mirror and device descriptor of a face array; *type receives the
  * effective boundary type (MGP_DIRICHLET / MGP_NEUMANN).  The face arrays of
