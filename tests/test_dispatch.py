@@ -33,7 +33,7 @@ PAIRS = ["sweep2", "sweep2_prolong", "sweep2_from_zero"]
 # with an out-of-range value left over can address
 @pytest.mark.parametrize("kind", PAIRS)
 @pytest.mark.parametrize("sfx,shape,n1,n2", [("f64", [129, 17, 33], 1025, 1025), ("f64", [129, 17, 33], 2049, 2049),
-                                             ("f32", [257, 17, 33], 1025, 1025), ("f64", [3, 9, 33], 4097, 16385)])
+                                             ("f32", [257, 33, 33], 1025, 1025), ("f64", [3, 9, 33], 4097, 16385)])
 def test_wide_windows_do_not_run_as_blocks(recorder, kind, sfx, shape, n1, n2):
     size = 8 if sfx == "f64" else 4
     wide = [n1 * n2, n2, 1]
@@ -169,3 +169,17 @@ def test_descent_kernel_by_size(recorder, shape, f64, f32):
              for sfx in ("f64", "f32")]
     names = [k[0][0] for rc, k in launch_recorder.record(recorder, calls)]
     assert all("k_resid_fw_" + want in name for name, want in zip(names, (f64, f32))), names
+
+
+# flat levels too large for blocks, on both sides of the rule: 16 rows in the box, 24
+# with the correction (FP32, Dirichlet faces)
+@pytest.mark.parametrize("kind,sfx,ny,bc,tile", [
+    ("sweep2", "f32", 16, "DDDDDD", False), ("sweep2", "f32", 17, "DDDDDD", True),
+    ("sweep2_from_zero", "f32", 16, "DDDDDD", False), ("sweep2_from_zero", "f32", 17, "DDDDDD", True),
+    ("sweep2_prolong", "f32", 23, "DDDDDD", False), ("sweep2_prolong", "f32", 25, "DDDDDD", True),
+    ("sweep2", "f64", 9, "DDDDDD", True), ("sweep2_prolong", "f64", 9, "DDDDDD", True),
+    ("sweep2", "f32", 9, "DDNDDD", True), ("sweep2_prolong", "f32", 9, "DDDDND", True)])
+def test_flat_levels_pair_by_wave_march(recorder, kind, sfx, ny, bc, tile):
+    call = sweep_call(kind, sfx, [513, ny + 2, 513], bc=bc)
+    ((rc, kernels),) = launch_recorder.record(recorder, [call])
+    assert rc == 0 and ("k_rbgs_tile" in kernels[0][0], "_wave" in kernels[0][0]) == (tile, not tile), kernels
